@@ -61,12 +61,13 @@ void launch_sub_chain(const int32_t* nn, int K, const int64_t* base, const int32
                       hipStream_t s);
 void launch_copy_ranges(const void* tasks, int64_t ntasks, const int32_t* members, int32_t* pool, hipStream_t s);
 void launch_negate(float* d, int64_t n, hipStream_t s);
-void launch_graph_search(const SearchArgs& a, int64_t grid, hipStream_t s);
+void launch_graph_search(const SearchArgs& a, int dtype, int64_t grid, hipStream_t s);
+void launch_search_totals_init(SearchTotals* t, hipStream_t s);
+size_t search_query_lds(const SearchArgs& a, int esz);
 void launch_invert_perm(const uint32_t* inv, int64_t N, uint32_t* perm, uint32_t* hits, int* err, hipStream_t s);
 void launch_permute_rows(const void* in, const uint32_t* inv, int64_t N, int64_t row_bytes, void* out, hipStream_t s);
 void launch_remap_table(const int32_t* ids, const uint32_t* inv, const uint32_t* perm, int64_t N, int M, int32_t* out,
                         hipStream_t s);
-size_t search_lds_bytes(int CC, int efr, int Dp, int H);
 void launch_sanitize(const int32_t* in, int64_t N, int M, uint32_t* out, hipStream_t s);
 void launch_init_flags(unsigned long long* bad_row, int* err, hipStream_t s);
 void launch_cagra_prune(const int32_t* G, int64_t N, int M, int K, uint32_t* out, unsigned long long* bad_row,
@@ -2651,86 +2652,113 @@ int gt_search(gt_ctx* ctx, const void* X, int64_t N, int32_t D, int dtype, const
         GT_REQUIRE(ef <= 2048, "ef must be <= 2048");
         GT_REQUIRE(p.metric == GT_METRIC_L2 || p.metric == GT_METRIC_IP, "unknown metric");
         GT_REQUIRE(N < (int64_t(1) << 31) - 1, "N must be < 2^31 - 1");
+        GT_REQUIRE(X != nullptr && N > 0 && D > 0, "empty dataset");
+        GT_REQUIRE(pad_dim(D) <= 1024, "dimension > 1024 is not supported by this build");
         Timer tt;
         Ctx c(ctx);
-        DevMatrix Xm = prepare(c, W_X, W_XRAW, W_NORMS, X, N, D, dtype);
         gt_search_stats st{};
         if (nq > 0) {
             GT_REQUIRE(Q != nullptr, "no queries");
-            DevMatrix Qm = prepare(c, W_C, W_CRAW, W_CNORMS, Q, nq, D, dtype);
-            const uint32_t* g = c.in<uint32_t>(W_IN, graph, static_cast<size_t>(N) * degree);
-            int E = n_entry;
-            const int32_t* d_ent = nullptr;
-            if (entries) {
-                GT_REQUIRE(n_entry >= 1 && n_entry <= 64, "1 <= n_entry <= 64");
-                d_ent = c.in<int32_t>(W_PROBE_I, entries, static_cast<size_t>(nq) * E);
-            } else {
-                E = p.num_entry;
-                GT_REQUIRE(E >= 1 && E <= 64, "1 <= num_entry <= 64");
-                // E draws per query from a splitmix64 stream, sorted and distinct
-                std::vector<int32_t> he(static_cast<size_t>(nq) * E, -1);
-                parallel_slices(nq, host_threads(), [&](int, int64_t lo, int64_t hi) {
-                    std::vector<int32_t> tmp(static_cast<size_t>(E));
-                    for (int64_t q = lo; q < hi; ++q) {
-                        for (int e = 0; e < E; ++e) {
-                            uint64_t z = p.seed + 0x9E3779B97F4A7C15ull * static_cast<uint64_t>(q * E + e + 1);
-                            z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
-                            z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
-                            z ^= z >> 31;
-                            tmp[static_cast<size_t>(e)] = static_cast<int32_t>(z % static_cast<uint64_t>(N));
-                        }
-                        std::sort(tmp.begin(), tmp.end());
-                        const auto end = std::unique(tmp.begin(), tmp.end());
-                        std::copy(tmp.begin(), end, he.begin() + q * E);
-                    }
-                });
-                int32_t* d = c.ws<int32_t>(W_PROBE_I, he.size());
-                c.h2d(d, he.data(), he.size() * sizeof(int32_t));
-                c.sync();   // he is released at the end of this scope
-                d_ent = d;
-            }
-            const size_t nr = static_cast<size_t>(nq) * p.topk;
-            int32_t* oi = c.in<int32_t>(W_IDS, out_ids, nr, false);
-            float* od = c.in<float>(W_D, out_d, nr, false);
-            int32_t* d_status = c.ws<int32_t>(W_FLAG, static_cast<size_t>(nq));
-            int32_t* d_exp = c.ws<int32_t>(W_DEG, static_cast<size_t>(nq));
-            int32_t* d_vis = c.ws<int32_t>(W_CUR, static_cast<size_t>(nq));
-
             SearchArgs a{};
-            a.X = Xm.data;
             a.N = N;
             a.D = D;
-            a.Dp = Xm.Dp;
-            a.graph = g;
+            // The search reads rows as they are stored: no copy of the base
+            // and no pass over it.  Byte rows beyond 256 dimensions (where
+            // the float chains may round) go through the float copy.
+            int rows_dtype = dtype;
+            const size_t es = dtype_size(dtype);
+            if (dtype == GT_DTYPE_F32 || D <= 256) {
+                a.X = c.in<uint8_t>(W_XRAW, static_cast<const uint8_t*>(X), static_cast<size_t>(N) * D * es);
+                a.Q = c.in<uint8_t>(W_CRAW, static_cast<const uint8_t*>(Q), static_cast<size_t>(nq) * D * es);
+                a.ld = D;
+            } else {
+                const DevMatrix Xm = prepare(c, W_X, W_XRAW, W_NORMS, X, N, D, dtype);
+                const DevMatrix Qm = prepare(c, W_C, W_CRAW, W_CNORMS, Q, nq, D, dtype);
+                a.X = Xm.data;
+                a.Q = Qm.data;
+                a.ld = Xm.Dp;
+                rows_dtype = GT_DTYPE_F32;
+            }
+            const int esz = static_cast<int>(dtype_size(rows_dtype));
+            a.graph = c.in<uint32_t>(W_IN, graph, static_cast<size_t>(N) * degree);
             a.deg = degree;
-            a.Q = Qm.data;
-            a.entries = d_ent;
-            a.n_entry = E;
-            a.n_run = nq;
+            if (entries) {
+                GT_REQUIRE(n_entry >= 1 && n_entry <= 64, "1 <= n_entry <= 64");
+                a.n_entry = n_entry;
+                a.entries = c.in<int32_t>(W_PROBE_I, entries, static_cast<size_t>(nq) * n_entry);
+            } else {
+                a.n_entry = p.num_entry;
+                GT_REQUIRE(a.n_entry >= 1 && a.n_entry <= 64, "1 <= num_entry <= 64");
+                a.seed = p.seed;
+            }
+            const size_t nr = static_cast<size_t>(nq) * p.topk;
+            a.out_ids = c.in<int32_t>(W_IDS, out_ids, nr, false);
+            a.out_d = c.in<float>(W_D, out_d, nr, false);
+            a.totals = c.ws<SearchTotals>(W_FLAG, 1);
+            a.redo = c.ws<int32_t>(W_DEG, static_cast<size_t>(nq));
             a.topk = p.topk;
             a.ef = ef;
             a.metric = p.metric;
             a.efr = static_cast<int32_t>(ceil_div(ef, 64) * 64);
             a.CC = a.efr + 256;
-            a.out_ids = oi;
-            a.out_d = od;
-            a.status = d_status;
-            a.expansions = d_exp;
-            a.visits = d_vis;
-            // visited set: an LDS hash table (a query visits up to about
-            // degree x ef points; the table holds 3/4 of its slots) or, when
-            // that table would leave fewer than five waves per CU (S2 at
-            // ef 200: one wave per SIMD, 19.0 ms against 10.7 ms), a bitmap
-            // of N bits per wave in HBM with a few KiB of LDS per wave
-            constexpr size_t kHashLdsMax = 32768;
+
+            // visited set: a table of H entries in LDS (16 bits each where
+            // the ids allow: an id's bits beyond the bucket number, at most
+            // 12, and four for the buckets passed over)
+            int id_bits = 1;
+            while (id_bits < 31 && (int64_t(1) << id_bits) < N) ++id_bits;
+            auto set_table = [&](int H) {
+                auto log2i = [](int x) { int l = 0; while ((1 << l) < x) ++l; return l; };
+                a.half = id_bits - log2i(H / 8) <= 12 ? 1 : 0;
+                a.buckets = a.half ? H / 8 : H / 4;
+                a.lbits = log2i(a.buckets);
+                a.nbits = std::max(id_bits, a.lbits);
+                a.vlimit = H - 3 * (H / 16);
+            };
+            // the room that a call may ask for: 64 KiB of candidates, best
+            // list, padded float query row and 4-byte table entries
+            auto fits = [&](int H) {
+                return static_cast<size_t>(a.CC) * 8 + static_cast<size_t>(a.efr) * 8 +
+                           static_cast<size_t>(pad_dim(D)) * 4 + static_cast<size_t>(H) * 4 <= 65536;
+            };
+            // by itself: room for 0.9 degree x ef points at 13/16 full (S2's
+            // queries visit 0.76 of degree x ef at ef 200, 0.9 at ef 64 on
+            // average), more where the queries leave LDS unused (a query
+            // that outgrows its table costs its time twice), unless that
+            // takes more than kTableLds, where too few waves fit a CU: then
+            // the bitmap of N bits per wave in HBM
+            constexpr size_t kTableLds = 40960;
             int H = p.visited_slots;
             bool bitmap_only = H == -1;
             if (H == 0) {
-                const int64_t want = static_cast<int64_t>(degree) * ef * 4 / 3;
+                const int64_t want = std::min<int64_t>(static_cast<int64_t>(degree) * ef * 10 / 9, N * 16 / 13 + 1);
+                const size_t spare = std::min<size_t>(kTableLds, 163840 / static_cast<size_t>(ceil_div(nq, 256)));
                 H = 512;
-                while (H < want && search_lds_bytes(a.CC, a.efr, a.Dp, 2 * H) <= 65536) H *= 2;
-                bitmap_only = search_lds_bytes(a.CC, a.efr, a.Dp, H) > kHashLdsMax;
+                set_table(H);
+                while (H < want && search_query_lds(a, esz) <= kTableLds) set_table(H *= 2);
+                bitmap_only = search_query_lds(a, esz) > kTableLds;
+                while (!bitmap_only && H < 2 * want) {
+                    set_table(2 * H);
+                    if (search_query_lds(a, esz) > spare) break;
+                    H *= 2;
+                }
             }
+            SearchTotals* h = c.c->pin_lloyd.as<SearchTotals>(1);
+            auto run = [&](int64_t grid) {
+                launch_search_totals_init(a.totals, c.s);
+                GT_HIP(hipEventRecord(c.c->ev0, c.s));
+                launch_graph_search(a, rows_dtype, grid, c.s);
+                GT_HIP(hipEventRecord(c.c->ev1, c.s));
+                c.d2h(h, a.totals, sizeof(*h));
+                c.sync();
+                float ms = 0.f;
+                GT_HIP(hipEventElapsedTime(&ms, c.c->ev0, c.c->ev1));
+                st.t_search += ms * 1e-3;
+                st.expansions += static_cast<int64_t>(h->expansions);
+                st.visited += static_cast<int64_t>(h->visits);
+                GT_REQUIRE(h->overflow == 0xFFFFFFFFu, "search: more candidates tie at the ef-th distance than fit (query " +
+                                                           std::to_string(h->overflow) + ")");
+            };
             // queries (all, or those that outgrew the on-chip table) on the
             // bitmap path: up to kBitmapWaves waves, each clearing its bitmap
             // after every query
@@ -2743,52 +2771,31 @@ int gt_search(gt_ctx* ctx, const void* X, int64_t N, int32_t D, int dtype, const
                 GT_HIP(hipMemsetAsync(bmp, 0, static_cast<size_t>(slots * words) * 4, c.s));
                 a.q_list = d_list;
                 a.n_run = n;
-                a.H = 0;
+                a.buckets = 0;
                 a.bitmap = bmp;
                 a.bm_words = words;
-                GT_REQUIRE(search_lds_bytes(a.CC, a.efr, a.Dp, 0) <= 65536, "ef / dimension too large for one query's LDS");
-                st.t_search += c.timed([&] { launch_graph_search(a, slots, c.s); });
+                GT_REQUIRE(fits(0), "ef / dimension too large for one query's LDS");
+                run(slots);
             };
-            std::vector<int32_t> hs(static_cast<size_t>(nq)), hx(static_cast<size_t>(nq)), hv(static_cast<size_t>(nq));
             if (bitmap_only) {
                 run_bitmap(nullptr, nq);
-                c.d2h(hs.data(), d_status, hs.size() * sizeof(int32_t));
-                c.sync();
-                for (int64_t q = 0; q < nq; ++q)
-                    GT_REQUIRE(hs[static_cast<size_t>(q)] == 0,
-                               "search: more candidates tie at the ef-th distance than fit (query " + std::to_string(q) + ")");
             } else {
                 GT_REQUIRE(H >= 512 && (H & (H - 1)) == 0, "visited_slots must be -1, 0 or a power of two >= 512");
-                GT_REQUIRE(search_lds_bytes(a.CC, a.efr, a.Dp, H) <= 65536, "ef / dimension too large for one query's LDS");
-                a.H = H;
-                st.t_search = c.timed([&] { launch_graph_search(a, nq, c.s); });
-                c.d2h(hs.data(), d_status, hs.size() * sizeof(int32_t));
-                c.sync();
-                std::vector<int32_t> redo;
-                for (int64_t q = 0; q < nq; ++q) {
-                    GT_REQUIRE(hs[static_cast<size_t>(q)] != 2,
-                               "search: more candidates tie at the ef-th distance than fit (query " + std::to_string(q) + ")");
-                    if (hs[static_cast<size_t>(q)] == 1) redo.push_back(static_cast<int32_t>(q));
-                }
-                if (!redo.empty()) {
-                    int32_t* d_redo = c.ws<int32_t>(W_QROWS, redo.size());
-                    c.h2d(d_redo, redo.data(), redo.size() * sizeof(int32_t));
-                    run_bitmap(d_redo, static_cast<int64_t>(redo.size()));
-                    c.d2h(hs.data(), d_status, hs.size() * sizeof(int32_t));
-                    c.sync();
-                    for (int32_t q : redo)
-                        GT_REQUIRE(hs[static_cast<size_t>(q)] == 0,
-                                   "search: more candidates tie at the ef-th distance than fit (query " + std::to_string(q) + ")");
-                    st.requeued = static_cast<int64_t>(redo.size());
+                GT_REQUIRE(p.visited_slots == 0 || fits(H), "ef / dimension too large for one query's LDS");
+                set_table(H);
+                a.n_run = nq;
+                run(nq);
+                if (h->n_redo > 0) {
+                    const int64_t n = h->n_redo;
+                    int32_t* list = c.ws<int32_t>(W_QROWS, static_cast<size_t>(n));
+                    c.d2d(list, a.redo, static_cast<size_t>(n) * sizeof(int32_t));
+                    run_bitmap(list, n);
+                    st.requeued = n;
                 }
             }
-            c.d2h(hx.data(), d_exp, hx.size() * sizeof(int32_t));
-            c.d2h(hv.data(), d_vis, hv.size() * sizeof(int32_t));
-            c.out(out_ids, oi, nr);
-            c.out(out_d, od, nr);
+            c.out(out_ids, a.out_ids, nr);
+            c.out(out_d, a.out_d, nr);
             c.sync();
-            for (int32_t x : hx) st.expansions += x;
-            for (int32_t x : hv) st.visited += x;
         }
         st.t_total = tt.sec();
         if (stats) *stats = st;

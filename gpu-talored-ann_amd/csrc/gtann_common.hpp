@@ -101,32 +101,43 @@ constexpr int kMaxChunkWords = 24;   // pools of up to 24 * 32 chunks (49,152 ro
 
 constexpr int kCollectCap = 256;   // candidate slots per query of a collect launch
 
+// What a search launch reports over all of its queries.
+struct SearchTotals {
+    unsigned long long expansions;   // of the queries that finished
+    unsigned long long visits;       // points whose distance they computed
+    uint32_t n_redo;                 // queries whose visited table filled (redo[0 .. n_redo))
+    uint32_t overflow;               // lowest query whose candidates did not fit, 0xFFFFFFFF if none
+};
+
 // Arguments of the graph search kernel (one wave per query).
 struct SearchArgs {
-    const float* X;           // base rows, stride Dp, zero padded
+    const void* X;            // base rows as stored, ld elements apart
+    int64_t ld;
     int64_t N;
     int32_t D;
-    int32_t Dp;
-    const uint32_t* graph;    // (N, deg); entries >= N are skipped
     int32_t deg;
-    const float* Q;           // query rows, stride Dp
-    const int32_t* entries;   // (nq, n_entry), processed in order; < 0 or >= N skipped
+    const uint32_t* graph;    // (N, deg); entries >= N are skipped
+    const void* Q;            // query rows, as X
+    const int32_t* entries;   // (nq, n_entry), processed in order; < 0 or >= N skipped; null: drawn from seed
+    uint64_t seed;
     int32_t n_entry;          // <= 64
+    int32_t topk;
     const int32_t* q_list;    // queries to run; nullptr = 0 .. n_run-1
     int64_t n_run;
-    int32_t topk;
     int32_t ef;
     int32_t metric;           // 0 = L2, 1 = inner product (key = -<q,x>)
-    int32_t H;                // LDS visited table slots (power of two >= 512); 0 = bitmap mode
     int32_t CC;               // candidate capacity (multiple of 64)
     int32_t efr;              // ef rounded up to a multiple of 64
+    int32_t buckets;          // visited table: 16-byte buckets (power of two); 0 = bitmap mode
+    int32_t half;             // its entries: 1 = eight 16-bit per bucket, 0 = four ids
+    int32_t nbits, lbits;     // bits of an id, of a bucket number
+    int32_t vlimit;           // visited points beyond which the query is left to the bitmap
     uint32_t* bitmap;         // bitmap mode: gridDim.x slots of bm_words words, zero on entry
     int64_t bm_words;
     int32_t* out_ids;         // (nq, topk)
     float* out_d;             // (nq, topk)
-    int32_t* status;          // (nq): 0 done, 1 visited table full, 2 candidate capacity exceeded
-    int32_t* expansions;      // (nq)
-    int32_t* visits;          // (nq): points whose distance was computed
+    SearchTotals* totals;
+    int32_t* redo;            // (nq)
 };
 
 inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }

@@ -322,8 +322,8 @@ typedef struct gt_search_params {
     int32_t metric;         /* GT_METRIC_L2 (the reference's only metric) or GT_METRIC_IP */
     uint64_t seed;          /* entry draw when `entries` is NULL */
     int32_t visited_slots;  /* visited set per query: 0 = automatic (an on-chip hash table, or an HBM
-                               bitmap of N bits per wave when the table would take more than 32 KiB
-                               of LDS); -1 = the HBM bitmap; else the on-chip table's slots (power of
+                               bitmap of N bits per wave when the query would take more than 40 KiB
+                               of LDS with it); -1 = the HBM bitmap; else the on-chip table's slots (power of
                                two >= 512), a query that outgrows it run again with the bitmap */
     int32_t reserved_;
 } gt_search_params;

@@ -30,6 +30,14 @@ void launch_knn_fused(const KnnArgs& a, hipStream_t stream);
 // knn_collect.hip
 bool knn_collect_supported(const KnnArgs& a);
 void launch_knn_collect_select(const KnnArgs& a, int64_t rows, hipStream_t stream);
+// knn_wide_collect.hip
+void launch_split_rows(const float* X, const float* nrm, const int32_t* members, int64_t N, int Dp, uint16_t* Xs,
+                       float* inv, unsigned int* bad, hipStream_t s);
+void launch_iota(int32_t* p, int64_t n, hipStream_t s);
+int wide_queries_per_block(int64_t n_queries);
+void launch_wide_collect(const KnnArgs& a, int qpb, const uint16_t* Xs, const float* inv, const int32_t* p_pos,
+                         hipStream_t s);
+void launch_collect_select(const KnnArgs& a, int64_t rows, hipStream_t stream);
 void launch_merge_partials(const int32_t* pids, const float* pd, int64_t nq, int splits, int M, int32_t* out_ids,
                            float* out_d, hipStream_t stream);
 bool resident_supported(const KnnArgs& a, int64_t np);
@@ -245,7 +253,7 @@ struct gt_ctx {
     hipStream_t stream = nullptr;
     std::string err;
     // named workspaces, grow-only (one slot per role, see gtann::Ws)
-    gtann::DevBuf ws[112];
+    gtann::DevBuf ws[128];
     gtann::HostBuf pinned[2];   // top-2 assignment downloads of two consecutive rounds
     gtann::HostBuf pin_lloyd;   // Lloyd steps: nearest centroids down, CSR up
     gtann::HostBuf pin_bucket[2];   // two-choice buckets of two consecutive rounds (uploaded for the device CSR)
@@ -257,9 +265,13 @@ struct gt_ctx {
     int64_t knn_launches = 0;   // bucketed-round launches of the current build
     double knn_pairs_done = 0;  // (query, pool row) pairs the collect kernels computed (chunk pruning skips the rest)
     uint64_t members_gen = 0;   // bucketing whose members W_MEMBERS holds (0: none)
+    uint64_t members_ver = 0;   // bumped whenever W_MEMBERS is written
     uint64_t data_gen = 0;      // bumped whenever W_X / W_NORMS are (re)written
     uint64_t screen_gen = 0;    // data_gen whose fp16 copy and scale W_XH / W_SQ hold (0: none)
     const float* screen_src = nullptr;
+    uint64_t split_gen = 0;     // data_gen whose fp16 pairs W_XSPLIT / W_XSINV hold (0: none)
+    uint64_t split_order = 0;   // members_ver of their order
+    bool split_bad = false;     // some |x|^2 of them is not finite
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     void* scratch = nullptr;    // this device's fixed scratch array (gt_optimize_noalloc), or null
     std::string scratch_err;    // why it is null
@@ -277,9 +289,10 @@ enum Ws {
     W_OOC_A, W_OOC_B, W_OOC_C, W_OOC_D, W_OOC_E, W_OOC_F, W_OOC_G, W_CR, W_CRNORMS,
     W_KM_TRAIN, W_KM_MIND, W_KM_FLAG, W_KM_SEL, W_KM_POS, W_KM_SUMS, W_KM_NEW, W_KM_PSI, W_KM_P, W_KM_PN, W_KM_P8,
     W_KM_PN8, W_KM_OI, W_KM_OD, W_CH8, W_CHN, W_CHR, W_CHCNT, W_PAIRS, W_TOP2A, W_TOP2B, W_BUCKETD, W_KEY2,
-    W_BYKEY, W_BKTD, W_BOFF, W_SUBPOS, W_TOP2H, W_RV1, W_RV1M, W_XH, W_UBASE, W_UROWS, W_UITEMS, W_TQ, W_SQ, W_PAIRS2, W_COUNT_
+    W_BYKEY, W_BKTD, W_BOFF, W_SUBPOS, W_TOP2H, W_RV1, W_RV1M, W_XH, W_UBASE, W_UROWS, W_UITEMS, W_TQ, W_SQ, W_PAIRS2, W_XSPLIT, W_XSINV,
+    W_XSBAD, W_XSIOTA, W_XSPOS, W_COUNT_
 };
-static_assert(W_COUNT_ <= 112, "workspace slots");
+static_assert(W_COUNT_ <= 128, "workspace slots");
 
 struct Ctx {
     gt_ctx* c;
@@ -1025,6 +1038,40 @@ static void sub_order_members(Ctx& c, const DevMatrix& X, const Buckets& b, int 
     int32_t* d_m2 = c.ws<int32_t>(W_MEMBERS2, static_cast<size_t>(N));
     launch_segment_sort(d_members, d_key, d_off, C, 2 * kSubSize, d_chain, d_sbase, d_m2, c.s);
     c.d2d(d_members, d_m2, static_cast<size_t>(N) * sizeof(int32_t));
+    ++c.c->members_ver;
+}
+
+// The rows of X split into two fp16 parts (knn_wide_collect.hip) in the order
+// of the member list, once per order; false where the copy and the launch's
+// candidate slots would not leave half of the free device memory, or the
+// inner product meets a row whose norm is not finite (the fp32 kernel then
+// takes the launch).
+static bool split_rows(Ctx& c, const DevMatrix& X, const int32_t* d_members, int64_t rows, int metric)
+{
+    const int64_t N = X.N, Np = ceil_div(N, int64_t(32)) * 32;
+    const size_t need = static_cast<size_t>(Np) * X.Dp * 4, cand = static_cast<size_t>(rows + kQueriesPerWave) * kCollectCap * 8;
+    const size_t more = (c.c->ws[W_XSPLIT].cap < need ? need : 0) + (c.c->ws[W_CAND].cap < cand ? cand : 0);
+    if (more > 0) {
+        size_t fr = 0, total = 0;
+        GT_HIP(hipMemGetInfo(&fr, &total));
+        if (more > fr / 2) return false;
+    }
+    uint16_t* xs = c.ws<uint16_t>(W_XSPLIT, need / 2);
+    float* inv = c.ws<float>(W_XSINV, static_cast<size_t>(N));
+    unsigned int* bad = c.ws<unsigned int>(W_XSBAD, 1);
+    if (c.c->split_gen != c.c->data_gen || c.c->split_order != c.c->members_ver) {
+        launch_split_rows(X.data, X.norms, d_members, N, X.Dp, xs, inv, bad, c.s);
+        c.c->split_gen = c.c->data_gen;
+        c.c->split_order = c.c->members_ver;
+        c.c->split_bad = false;
+        if (metric == GT_METRIC_IP) {
+            unsigned int h = 0;
+            c.d2h(&h, bad, sizeof(h));
+            c.sync();
+            c.c->split_bad = h > 0;
+        }
+    }
+    return !c.c->split_bad;
 }
 
 // One round of pooled kNN into (out_ids, out_d) rows by global id.
@@ -1083,6 +1130,7 @@ static double bucketed_round(Ctx& c, const DevMatrix& X, const Buckets& b, int M
         c.h2d(d_members, b.members.data(), static_cast<size_t>(N) * sizeof(int32_t));
         if (b.uploaded) GT_HIP(hipEventRecord(b.uploaded, c.s));
         c.c->members_gen = b.gen;
+        ++c.c->members_ver;
     }
     // members by nearest sub-centroid: for the unseeded pass (its threshold
     // tightens within a few tiles), and for seeded passes that prune chunks
@@ -1101,14 +1149,26 @@ static double bucketed_round(Ctx& c, const DevMatrix& X, const Buckets& b, int M
         pairs_all += static_cast<double>(b.offsets[static_cast<size_t>(bb + 1)] - b.offsets[static_cast<size_t>(bb)]) *
                      static_cast<double>(pool_cnt[static_cast<size_t>(bb)]);
     const int scr = c.c->dbg.knn_screen;
-    const bool want_screen = c.c->dbg.knn_collect != 0 && !use_i8(X, X, metric) &&
+    const bool want_screen = c.c->dbg.knn_collect != 0 && !use_i8(X, X, metric) && X.Dp <= 160 &&
                              (scr == 2 || (scr == 1 && pairs_all >= static_cast<double>(int64_t(1) << 27)));
     const bool sub_ordered = own && !compact && c.c->dbg.sub_order != 0 && (!seed_d || want_prune || want_screen);
     if (sub_ordered) sub_order_members(c, X, b, metric, d_members);
+    // fp32 rows longer than 160: collect on the fp16 matrix cores over rows
+    // split in two, 256 or 128 queries per block (lists of 5..128 keys)
+    const bool wide = c.c->dbg.knn_collect != 0 && !use_i8(X, X, metric) && X.Dp > 160 && M > 4 && M <= 128 &&
+                      split_rows(c, X, d_members, rows, metric);
+    const int qstep = wide ? wide_queries_per_block(rows) : kQueriesPerBlock;
     CopyTaskH* d_tasks = c.ws<CopyTaskH>(W_TASKS, tasks.size());
     c.h2d(d_tasks, tasks.data(), tasks.size() * sizeof(CopyTaskH));
     int32_t* d_pool = c.ws<int32_t>(W_POOL, static_cast<size_t>(std::max<int64_t>(total, 1)));
     launch_copy_ranges(d_tasks, static_cast<int64_t>(tasks.size()), d_members, d_pool, c.s);
+    int32_t* d_ppos = nullptr;   // wide: the pool entries' positions in the member list
+    if (wide) {
+        int32_t* iota = c.ws<int32_t>(W_XSIOTA, static_cast<size_t>(N));
+        launch_iota(iota, N, c.s);
+        d_ppos = c.ws<int32_t>(W_XSPOS, static_cast<size_t>(std::max<int64_t>(total, 1)));
+        launch_copy_ranges(d_tasks, static_cast<int64_t>(tasks.size()), iota, d_ppos, c.s);
+    }
 
     std::vector<std::vector<WorkItem>> groups(static_cast<size_t>(C));
     int64_t mp = 0, mb = 0;
@@ -1119,18 +1179,18 @@ static double bucketed_round(Ctx& c, const DevMatrix& X, const Buckets& b, int M
         mp = std::max(mp, npb);
         mb = std::max(mb, nqb);
         pr += static_cast<double>(nqb) * static_cast<double>(npb);
-        for (int64_t t = 0; t < nqb; t += kQueriesPerBlock) {
+        for (int64_t t = 0; t < nqb; t += qstep) {
             WorkItem it;
             it.q_begin = q0 + t;
-            it.q_count = static_cast<int32_t>(std::min<int64_t>(kQueriesPerBlock, nqb - t));
+            it.q_count = static_cast<int32_t>(std::min<int64_t>(qstep, nqb - t));
             it.p_begin = p0;
             it.p_count = static_cast<int32_t>(npb);
             // own bucket = first pool segment: start the scan at these queries'
             // own rows (members are ordered so that neighbours sit close by),
             // for the sub-ordered unseeded pass one sub-cluster earlier (the
             // chain's previous sub-cluster lies there)
-            int64_t rot = own && npb > 0 ? t : 0;
-            if (sub_ordered && !seed_d && nqb >= 2 * kSubSize && npb >= kSubSize) rot = (t - kSubSize + npb) % npb;   // >= 0
+            int64_t rot = own && npb > 0 && !wide ? t : 0;
+            if (sub_ordered && !wide && !seed_d && nqb >= 2 * kSubSize && npb >= kSubSize) rot = (t - kSubSize + npb) % npb;   // >= 0
             GT_REQUIRE(rot >= 0 && (npb == 0 || rot < npb), "pool rotation out of range");
             it.p_rot = static_cast<int32_t>(rot);
             it.out_base = compact ? q0 - qbase + t : -1;
@@ -1159,7 +1219,7 @@ static double bucketed_round(Ctx& c, const DevMatrix& X, const Buckets& b, int M
     a.out_d = out_d;
     // lists of at most 64 keys on int8 rows: collect + select (every point
     // is the query of exactly one work item, so rows = N)
-    const bool collect = c.c->dbg.knn_collect != 0 && knn_collect_supported(a);
+    const bool collect = wide || (c.c->dbg.knn_collect != 0 && knn_collect_supported(a));
     if (collect) {
         // (+ one wave's rows of slack: the selection reads whole groups of
         // 32 rows and masks the rows past the last)
@@ -1173,7 +1233,7 @@ static double bucketed_round(Ctx& c, const DevMatrix& X, const Buckets& b, int M
         GT_HIP(hipMemsetAsync(a.pairs_done, 0, sizeof(unsigned long long), c.s));
         // a seeded pass given its running table's ids: the new lists merge
         // into (run_ids, seed_d) in place
-        if (run_ids && seed_d) {
+        if (run_ids && seed_d && M <= 64) {
             a.run_ids = run_ids;
             a.run_d = const_cast<float*>(seed_d);
             a.hl_rows = c.ws<int32_t>(W_HLIST, static_cast<size_t>(rows));
@@ -1286,8 +1346,14 @@ static double bucketed_round(Ctx& c, const DevMatrix& X, const Buckets& b, int M
                           metric, seed_d, M, M,
                           screen_window, d_tq, d_urows, d_uitems, a.pairs_done, c.s);
         }
-        if (collect) launch_knn_collect_select(a, rows, c.s);
-        else launch_knn_fused(a, c.s);
+        if (wide) {
+            launch_wide_collect(a, qstep, c.ws<uint16_t>(W_XSPLIT, 0), c.ws<float>(W_XSINV, 0), d_ppos, c.s);
+            launch_collect_select(a, rows, c.s);
+        } else if (collect) {
+            launch_knn_collect_select(a, rows, c.s);
+        } else {
+            launch_knn_fused(a, c.s);
+        }
     });
     if (tr.on && screen) {
         std::vector<WorkItem> ui(items.size());
@@ -1557,6 +1623,7 @@ static void bucket_device(Ctx& c, const DevMatrix& X, int64_t C, int nprobe, int
         int64_t* hoff = reinterpret_cast<int64_t*>(pin + 2 * s4);
         int32_t* d_mem = c.ws<int32_t>(W_MEMBERS, static_cast<size_t>(S));
         c.c->members_gen = 0;   // W_MEMBERS no longer holds a bucketing's members
+        ++c.c->members_ver;
         int64_t* d_off = c.ws<int64_t>(W_OFF, static_cast<size_t>(C + 1));
         std::vector<int64_t> off;
         // the CSR on the device: no host round trip per iteration
@@ -3547,6 +3614,7 @@ int gt_build_graph_ex(gt_ctx* ctx, const void* X, int64_t N, int32_t D, int dtyp
             c.sync();
             GT_REQUIRE(b.offsets[0] == 0 && b.offsets[static_cast<size_t>(C)] == N, "device bucket CSR");
             c.c->members_gen = b.gen;   // W_MEMBERS holds these buckets' members
+            ++c.c->members_ver;
             st.t_bucketing += tc.sec();
         };
         device_part(0);

@@ -22,7 +22,7 @@
 // knn_select_kernel sorts each query's candidates into its top-M list: two
 // lanes per query merge 32 keys at a time into a sorted register list
 // (pair_merge32).
-#include "knn_device.hpp"
+#include "collect_device.hpp"
 
 #include <climits>
 #include <cstdlib>
@@ -38,21 +38,6 @@ __device__ __forceinline__ int window_tiles(const KnnArgs& a)
 {
     return a.window_tiles > 0 ? min(a.window_tiles, kWindowMax) & ~1 : kWindow;
 }
-
-// Per-wave staging of a tile's candidates: every lane's 16 accumulators
-// (16-byte chunks swizzled by lane so that a wave's 128-bit stores spread
-// over the banks), one 16-bit code (lane << 4 | element) per accumulator at
-// or above its lane's pass floor (plus a spare slot per lane), the wave's
-// queries' slot counters and the query state the dense pass reads.
-constexpr int kCodeSpare = 64 * 16;   // first of the 64 per-lane spare code slots
-
-struct CollectWave {
-    int32_t stash[64 * 16];
-    uint16_t code[kCodeSpare + 64];
-    int32_t qcnt[kQueriesPerWave];
-    float4 qst[kQueriesPerWave];          // |q|^2, threshold, threshold id (bits), self (bits)
-    int64_t qrow_out[kQueriesPerWave];    // output row
-};
 
 constexpr int kStageTiles = 2;                       // tiles (of kPoolTile pool rows) per pipeline stage
 constexpr int kStageRows = kPoolTile * kStageTiles;
@@ -73,82 +58,6 @@ struct CollectSmem {
     int32_t nlist;
 };
 static_assert(kChunkRows == kStageRows, "a pruning chunk is one stage of pool rows");
-
-__device__ __forceinline__ int stash_index(int lane, int r)
-{
-    return lane * 16 + (((r >> 2) ^ ((lane >> 1) & 3)) << 2) + (r & 3);
-}
-
-// Per-lane view of one query (lanes j and j + 32 hold identical copies).
-struct CollectState {
-    float thr;          // a key passes iff (d, id) <= (thr, thr_id)
-    uint32_t thr_id;    // 0xffffffff: every id at distance thr
-    int32_t cnt;        // keys in the query's slots
-    int32_t self;       // id that must not be kept (the query itself), -2 if none
-    int64_t orow;       // output row
-};
-
-__device__ __forceinline__ bool key_passes(float d, int32_t id, const CollectState& st)
-{
-    return d < st.thr || (d == st.thr && static_cast<uint32_t>(id) <= st.thr_id);
-}
-
-// Keeps the M smallest of query q's cnt (> M) keys in its slots and makes the
-// M-th its threshold.  Called by all 64 lanes; q is uniform.
-__device__ __forceinline__ void collect_compact(const KnnArgs& a, int lane, int q, CollectState& st)
-{
-    const int cntq = __builtin_amdgcn_readlane(st.cnt, q);
-    const int64_t orow = static_cast<int64_t>(
-        (static_cast<uint64_t>(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(st.orow >> 32), q))) << 32) |
-        static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(st.orow), q)));
-    uint64_t* slots = a.cand + orow * kCollectCap;
-    // the slots were stored by lanes q and q + 32: complete, then visible to
-    // the wave (workgroup-scope loads)
-    wait_vmem();
-    wave_sync();
-    constexpr int KPL = kCollectCap / 64;   // slots per lane
-    static_assert(kCollectCap % 64 == 0, "whole slots per lane");
-    uint64_t k[KPL];
-#pragma unroll
-    for (int i = 0; i < KPL; ++i)
-        k[i] = lane + 64 * i < cntq
-                   ? __hip_atomic_load(slots + lane + 64 * i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)
-                   : kNoKey;
-    // the M-th smallest key: the largest K with fewer than M keys below it
-    const int M = a.M;
-    uint64_t K = 0;
-    for (int b = 63; b >= 0; --b) {
-        const uint64_t t = K | (1ull << b);
-        int below = 0;
-#pragma unroll
-        for (int i = 0; i < KPL; ++i) below += __popcll(__ballot(k[i] < t));
-        if (below < M) K = t;
-    }
-    const uint64_t lt = (1ull << lane) - 1ull;
-    int base = 0;
-#pragma unroll
-    for (int i = 0; i < KPL; ++i) {
-        const bool p = k[i] <= K;
-        const uint64_t m = __ballot(p);
-        if (p) slots[base + __popcll(m & lt)] = k[i];
-        base += __popcll(m);
-    }
-    if ((lane & 31) == q) {
-        st.cnt = M;
-        st.thr = o2f(static_cast<uint32_t>(K >> 32));
-        st.thr_id = static_cast<uint32_t>(K);
-    }
-    if (a.stats && lane == 0) atomicAdd(a.stats + 1, 1ull);
-}
-
-// The query state the dense pass reads, published by lanes 0..31.
-__device__ __forceinline__ void publish_state(CollectWave& W, int lane, bool qvalid, float qn, const CollectState& st)
-{
-    if (lane < kQueriesPerWave) {
-        W.qst[lane] = make_float4(qn, qvalid ? st.thr : -INFINITY, __uint_as_float(st.thr_id), __int_as_float(st.self));
-        W.qrow_out[lane] = st.orow;
-    }
-}
 
 // One finished 32x32 tile of the collect scan: acc holds v = dot -
 // floor(|p|^2 / 2) (L2) or dot (IP) for the pool rows with norms tn, ids tr
@@ -604,9 +513,7 @@ __device__ __forceinline__ void f32_tile_keys(const floatx16& acc, const float* 
     }
 }
 
-// collect_tile for fp32 keys: the stash holds the keys themselves; a code is
-// written for every key at or below the query's threshold, and the exact
-// (key, id) test and the append are made per code.
+// collect_tile for fp32 rows.
 template <int METRIC>
 __device__ __forceinline__ void collect_tile_f32(const KnnArgs& a, CollectWave& W, const floatx16& acc,
                                                  const float* tn, const int32_t* tr, int lane, int h, bool qvalid,
@@ -614,57 +521,7 @@ __device__ __forceinline__ void collect_tile_f32(const KnnArgs& a, CollectWave& 
 {
     float d[16];
     f32_tile_keys<METRIC>(acc, tn, h, qn, d);
-    float dmin = d[0];
-#pragma unroll
-    for (int r = 1; r < 16; ++r) dmin = fminf(dmin, d[r]);
-    if (!__ballot(dmin <= st.thr)) return;
-    uint64_t need = __ballot(qvalid && st.cnt > kCollectCap - 2 * 16) & 0xffffffffull;
-    if (need) {
-        while (need) {
-            const int q = __ffsll(static_cast<unsigned long long>(need)) - 1;
-            need &= need - 1;
-            collect_compact(a, lane, q, st);
-        }
-        publish_state(W, lane, qvalid, qn, st);
-    }
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
-        *reinterpret_cast<int4*>(&W.stash[stash_index(lane, 4 * c)]) =
-            make_int4(__float_as_int(d[4 * c]), __float_as_int(d[4 * c + 1]), __float_as_int(d[4 * c + 2]),
-                      __float_as_int(d[4 * c + 3]));
-    if (lane < kQueriesPerWave) W.qcnt[lane] = st.cnt;
-    int c = 0;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) c += d[r] <= st.thr ? 1 : 0;
-    const int incl = wave_incl_scan(c);
-    const int total = __builtin_amdgcn_readlane(incl, 63);
-    int pos = incl - c;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const bool p = d[r] <= st.thr;
-        W.code[p ? pos : kCodeSpare + lane] = static_cast<uint16_t>((lane << 4) | r);
-        pos += p ? 1 : 0;
-    }
-    wave_sync();
-    for (int k = lane; k - lane < total; k += 64) {
-        if (k < total) {
-            const int code = W.code[k];
-            const int src = code >> 4, r = code & 15;
-            const float dk = __int_as_float(W.stash[stash_index(src, r)]);
-            const int q = src & 31;
-            const int row = 8 * (r >> 2) + 4 * (src >> 5) + (r & 3);
-            const int32_t id = tr[row];
-            const float4 Q = W.qst[q];
-            const bool ok = id >= 0 && id != __float_as_int(Q.w) &&
-                            (dk < Q.y || (dk == Q.y && static_cast<uint32_t>(id) <= __float_as_uint(Q.z)));
-            if (ok) {
-                const int slot = atomicAdd(&W.qcnt[q], 1);
-                a.cand[W.qrow_out[q] * kCollectCap + slot] = pack_key(dk, id);
-            }
-        }
-    }
-    wave_sync();
-    st.cnt = W.qcnt[lane & 31];
+    collect_keys_f32(a, W, d, tr, lane, qvalid, qn, st);
 }
 
 // window_tile for fp32 keys.
@@ -1427,6 +1284,11 @@ void launch_chunk_bounds(const int8_t* X8, int Dp, const int32_t* pool, const in
 
 // ------------------------------------------------------------ host side
 
+// knn_wide_collect.hip
+void launch_sort_select(const uint64_t* cand, const int32_t* cnt, int64_t rows, int M, int32_t* out_ids, float* out_d,
+                        hipStream_t s);
+void launch_collect_select(const KnnArgs& a, int64_t rows, hipStream_t stream);
+
 // Shapes the collect + select kernels take (the context's knn_collect
 // option can keep the merging kernel for every list; same results)
 bool knn_collect_supported(const KnnArgs& a)
@@ -1482,8 +1344,20 @@ void launch_knn_collect_select(const KnnArgs& a, int64_t rows, hipStream_t strea
         else launch_collect_f32_metric<1>(a, grid, stream);
         GT_HIP(hipGetLastError());
     }
+    launch_collect_select(a, rows, stream);
+}
+
+// The collected keys of rows [0, rows) into their lists: selected into
+// (out_ids, out_d), or merged into the running table.
+void launch_collect_select(const KnnArgs& a, int64_t rows, hipStream_t stream)
+{
     if (rows <= 0) return;
     const bool merge = a.run_ids != nullptr;
+    GT_REQUIRE(a.M >= 1 && (a.M <= 64 || (a.M <= 128 && !merge)), "collect selection: list length");
+    if (a.M > 64) {
+        launch_sort_select(a.cand, a.cand_cnt, rows, a.M, a.out_ids, a.out_d, stream);
+        return;
+    }
     GT_REQUIRE(!merge || (a.run_d && a.seed_d && a.seed_ld == a.M), "collect merge: running table missing");
     const dim3 sgrid(static_cast<unsigned>(ceil_div(rows, kQueriesPerBlock)));
     const dim3 mgrid(static_cast<unsigned>(ceil_div(rows, int64_t(64) * kWaves)));

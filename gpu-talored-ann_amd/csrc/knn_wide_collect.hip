@@ -1,0 +1,489 @@
+// knn_wide_collect.hip -- collect + select kNN for fp32 rows longer than 160
+// floats, the contraction on the fp16 matrix cores over rows split in two
+// (src/bucket.cu:4101-4265 top-M semantics: self excluded, (-1, +inf)
+// padding, ties by id).
+//
+// The split.  Row x is scaled by a power of two of its own, 2^k with
+// max |x_i| 2^k in [2^14, 2^15), and every element written as h + m: h the
+// fp16 nearest to it, m the fp16 nearest to the rest.  h keeps 11 bits and a
+// sign, m the next 11, so h + m is the fp32 element to within half of its
+// last bit (2^-24 of the element; where m is subnormal, flushed or not,
+// within 2^-29 of the row's largest).  A dot product is the sum of h h, h m and m h
+// products, each exact in the fp32 accumulator (v_mfma_f32_32x32x16_f16);
+// the m m products left out are at most 2^-24 of their terms.  Both are
+// below the roundings of an fp32 sum over D terms: measured against 64 bits
+// on D 161..1024 (tests/test_gpu_wide_split.py) the distances are closer than
+// those of the fp32 kernel (knn_wide_kernel).  Integer-valued rows below 2^11
+// have m = 0 and give exact sums.
+// A row with an element that is not finite has a norm that is not finite
+// either: its L2 keys are +inf or NaN, which no list takes, whatever its dot
+// products (the inner product of such rows stays on the fp32 kernel).
+//
+// Three fp16 products cost 3/16 of one fp32 product of the fp32 matrix cores,
+// and h and m take the fp32 row's bytes, so what bounds the kernel is moving
+// rows, not multiplying: a block is 8 waves with 256 queries (32 per wave,
+// read from L2 chunk by chunk) against 256 pool rows at a time (32-dimension
+// chunks double-buffered in LDS, shared by the waves; 8 accumulator tiles of
+// 32 x 32 per wave), 64 KiB of rows per 65,536 x 32 multiply-adds.  Launches
+// with fewer blocks than the chip has CUs take 4 waves and 128 queries.
+//
+// Keys at or below a query's threshold go to its candidate slots in HBM as in
+// knn_collect.hip.  An unseeded pass first bounds each query's M-th smallest
+// key by bisection over the 256 keys of the first pool tile, which the lane
+// pair holds in registers.
+#include "collect_device.hpp"
+
+#include <algorithm>
+
+namespace gtann {
+
+typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
+typedef _Float16 halfx4 __attribute__((ext_vector_type(4)));
+
+constexpr int kSplitChunk = 32;                   // dimensions per chunk: 32 h, then 32 m
+constexpr int kSplitRows = 192;                   // pool rows per tile
+constexpr int kSplitTiles = kSplitRows / kPoolTile;
+constexpr int kGroup = 1;                         // tiles multiplied at a time
+constexpr int kSplitStride = 2 * kSplitChunk + 8; // halves per LDS row: 16 rows' same pieces fill the banks once
+
+// Where the split copy holds chunk c of the row at position p of the member
+// list: groups of 32 positions, chunk-major, so that a tile's chunk is a few
+// whole 4 KiB pieces (by row id, a 128-byte piece of a row in 512 places per
+// chunk, the launch took 2.1 times as long).
+__device__ __forceinline__ int64_t split_at(int64_t p, int c, int nch)
+{
+    return (((p >> 5) * nch + c) * 32 + (p & 31)) * 2 * kSplitChunk;
+}
+
+// The rows X[members[p]] (stride Dp) to Xs at their positions p: per row and
+// chunk 32 h, then 32 m; inv[p] = 2^-k.  *bad counts rows whose |x|^2 is not
+// finite.  One wave per position.
+__global__ void __launch_bounds__(256) split_rows_kernel(const float* __restrict__ X, const float* __restrict__ nrm,
+                                                         const int32_t* __restrict__ members, int64_t N, int Dp,
+                                                         _Float16* __restrict__ Xs, float* __restrict__ inv,
+                                                         unsigned int* __restrict__ bad)
+{
+    const int lane = threadIdx.x & 63;
+    const int64_t pos = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
+    if (pos >= N) return;
+    const int64_t row = members[pos];
+    const float4* x = reinterpret_cast<const float4*>(X + row * Dp);
+    const int n4 = Dp >> 2;
+    float4 v[4];                                   // Dp <= 1024: four float4 per lane
+    float mx = 0.f;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        v[t] = lane + 64 * t < n4 ? x[lane + 64 * t] : make_float4(0.f, 0.f, 0.f, 0.f);
+        mx = fmaxf(fmaxf(fmaxf(mx, fabsf(v[t].x)), fmaxf(fabsf(v[t].y), fabsf(v[t].z))), fabsf(v[t].w));
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+    int e = 0;
+    const bool finite = mx < INFINITY;
+    if (finite && mx > 0.f) frexpf(mx, &e);        // mx < 2^e
+    const int k = finite && mx > 0.f ? 15 - e : 0;
+    auto scaled = [&](float y) -> float { return finite ? ldexpf(y, k) : 0.f; };
+    const int nch = Dp / kSplitChunk;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        const int q = lane + 64 * t;
+        if (q < n4) {
+            const float y[4] = {scaled(v[t].x), scaled(v[t].y), scaled(v[t].z), scaled(v[t].w)};
+            halfx4 h, m;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                h[i] = static_cast<_Float16>(y[i]);
+                m[i] = static_cast<_Float16>(y[i] - static_cast<float>(h[i]));
+            }
+            const int d = 4 * q;                   // dims d .. d + 3 of chunk d / 32
+            _Float16* c = Xs + split_at(pos, d / kSplitChunk, nch) + d % kSplitChunk;
+            *reinterpret_cast<halfx4*>(c) = h;
+            *reinterpret_cast<halfx4*>(c + kSplitChunk) = m;
+        }
+    }
+    if (lane == 0) {
+        inv[pos] = ldexpf(1.f, -k);
+        if (!(nrm[row] < INFINITY)) atomicAdd(bad, 1u);
+    }
+}
+
+__global__ void split_clear_kernel(unsigned int* bad) { *bad = 0u; }
+
+void launch_split_rows(const float* X, const float* nrm, const int32_t* members, int64_t N, int Dp, uint16_t* Xs,
+                       float* inv, unsigned int* bad, hipStream_t s)
+{
+    GT_REQUIRE(Dp % kSplitChunk == 0 && Dp <= 1024, "split rows: padded dimension");
+    hipLaunchKernelGGL(split_clear_kernel, dim3(1), dim3(1), 0, s, bad);
+    if (N > 0)
+        hipLaunchKernelGGL(split_rows_kernel, dim3(static_cast<unsigned>(ceil_div(N, int64_t(4)))), dim3(256), 0, s, X,
+                           nrm, members, N, Dp, reinterpret_cast<_Float16*>(Xs), inv, bad);
+    GT_HIP(hipGetLastError());
+}
+
+__global__ void __launch_bounds__(256) iota_kernel(int32_t* p, int64_t n)
+{
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+    if (i < n) p[i] = static_cast<int32_t>(i);
+}
+
+void launch_iota(int32_t* p, int64_t n, hipStream_t s)
+{
+    if (n <= 0) return;
+    hipLaunchKernelGGL(iota_kernel, dim3(static_cast<unsigned>(ceil_div(n, int64_t(256)))), dim3(256), 0, s, p, n);
+    GT_HIP(hipGetLastError());
+}
+
+template <int NW>
+struct WideCollectSmem {
+    _Float16 tile[2][kSplitRows][kSplitStride];
+    float tnorm[2][kSplitRows];     // |p|^2 (L2) or 0 (IP); +inf past the slice end
+    float tinv[2][kSplitRows];      // 2^-k of the row
+    int32_t trow[2][kSplitRows];    // pool row id, -1 past the slice end
+    CollectWave wv[NW];
+};
+
+template <int METRIC, int NW>
+__global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW == 8 ? 2 : 1)))
+knn_wide_collect_kernel(KnnArgs a, const _Float16* __restrict__ Xs, const float* __restrict__ inv,
+                        const int32_t* __restrict__ p_pos)
+{
+    extern __shared__ __align__(16) unsigned char smem[];
+    WideCollectSmem<NW>& sm = *reinterpret_cast<WideCollectSmem<NW>*>(smem);
+    constexpr int T = 64 * NW;
+    constexpr int PT = kSplitRows * 8 / T;          // 16-byte pieces of a chunk's rows per thread
+    static_assert(PT * T == kSplitRows * 8, "whole pieces");
+    constexpr int RS = T / 8;                       // rows between a thread's pieces
+
+    const int per = a.n_items / 8;
+    const int item_idx = static_cast<int>(blockIdx.x % 8) * per + static_cast<int>(blockIdx.x / 8);
+    if (item_idx >= a.n_items) return;
+    const WorkItem it = a.items[item_idx];
+    if (it.q_count <= 0) return;
+
+    const int Dp = a.Dp;
+    const int nch = Dp / kSplitChunk;
+    const int tid = threadIdx.x;
+    const int w = tid >> 6, lane = tid & 63, j = lane & 31, h = lane >> 5;
+    const int qlocal = w * kQueriesPerWave + j;
+    const bool qvalid = qlocal < it.q_count;
+    const int64_t qi = it.q_begin + qlocal;
+    const int32_t qrow = qvalid ? (a.q_rows ? a.q_rows[qi] : static_cast<int32_t>(qi)) : 0;
+    const float qn = (qvalid && METRIC == 0) ? a.nq[qrow] : 0.f;
+    const int64_t qpos = qvalid ? qi : it.q_begin;
+    const float qinv = inv[qpos];
+
+    CollectState st;
+    float seed = FLT_MAX;
+    // the seed is read from the output row (the query row unless the item has an out_base)
+    const int64_t orow = it.out_base >= 0 ? it.out_base + qlocal : static_cast<int64_t>(qrow);
+    if (qvalid && a.seed_d) seed = fminf(a.seed_d[orow * a.seed_ld + a.seed_ld - 1], FLT_MAX);
+    st.thr = qvalid ? seed : -INFINITY;
+    st.thr_id = 0xffffffffu;
+    st.cnt = 0;
+    st.self = a.exclude_self ? qrow : -2;
+    st.orow = orow;
+    CollectWave& W = sm.wv[w];
+    publish_state(W, lane, qvalid, qn, st);
+
+    const int pcount = it.p_count;
+    const int nst = (pcount + kSplitRows - 1) / kSplitRows;
+    // the pool-list entry scanned at p (< pcount)
+    auto pool_at = [&](int p) -> int64_t {
+        p += it.p_rot;
+        if (p >= pcount) p -= pcount;
+        return it.p_begin + p;
+    };
+
+    // thread tid stages 16-byte piece tid % 8 of rows tid / 8 + RS u (rows past
+    // the slice hold the last row's values: their norm is +inf and their id -1)
+    const int piece = tid & 7, r0 = tid >> 3;
+    int32_t rid[PT], rid_n[PT];   // their positions in the member list
+    uint4 pre[PT];
+    auto set_ids = [&](int stile, int32_t (&ids)[PT]) {
+#pragma unroll
+        for (int u = 0; u < PT; ++u) ids[u] = p_pos[pool_at(min(stile * kSplitRows + r0 + RS * u, pcount - 1))];
+    };
+    auto load_pool = [&](bool next, int c) {
+#pragma unroll
+        for (int u = 0; u < PT; ++u) {
+            const int32_t p = next ? rid_n[u] : rid[u];
+            const uint4 v = *reinterpret_cast<const uint4*>(Xs + split_at(p, c, nch) + 8 * piece);
+            pre[u] = make_uint4(v.x, v.y, v.z, v.w);
+        }
+    };
+    auto store_pool = [&](int buf) {
+#pragma unroll
+        for (int u = 0; u < PT; ++u) *reinterpret_cast<uint4*>(&sm.tile[buf][r0 + RS * u][8 * piece]) = pre[u];
+    };
+    // the query's chunk: h of dims 8h.., 16 + 8h.., then m
+    halfx8 qc[4], qx[4];
+    auto load_q = [&](int c, halfx8 (&dst)[4]) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) dst[s] = *reinterpret_cast<const halfx8*>(Xs + split_at(qpos, c, nch) + 8 * h + 16 * s);
+    };
+    // ids, norms and scales of tile stile's row tid
+    auto tile_meta = [&](int stile, int32_t& id, float& n, float& iv) {
+        id = -1;
+        n = INFINITY;
+        iv = 1.f;
+        const int p = stile * kSplitRows + tid;
+        if (tid < kSplitRows && p < pcount) {
+            const int64_t pl = pool_at(p);
+            id = a.p_rows[pl];
+            n = METRIC == 0 ? a.np[id] : 0.f;
+            iv = inv[p_pos[pl]];
+        }
+    };
+    static_assert(T >= kSplitRows || T == 256, "one row's ids per thread");
+
+    if (nst > 0) {
+        set_ids(0, rid);
+        set_ids(1, rid_n);
+        int32_t nrow;
+        float nnrm, ninv;
+        tile_meta(0, nrow, nnrm, ninv);
+        if (tid < kSplitRows) {
+            sm.trow[0][tid] = nrow;
+            sm.tnorm[0][tid] = nnrm;
+            sm.tinv[0][tid] = ninv;
+        }
+        load_pool(false, 0);
+        store_pool(0);
+        load_q(0, qc);
+        __syncthreads();
+    }
+
+    int g = 0;
+    for (int stile = 0; stile < nst; ++stile) {
+        floatx16 acc[kSplitTiles];
+#pragma unroll
+        for (int u = 0; u < kSplitTiles; ++u)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[u][r] = 0.f;
+        int32_t nrow;
+        float nnrm, ninv;
+        tile_meta(stile + 1, nrow, nnrm, ninv);
+#pragma unroll 1
+        for (int c = 0; c < nch; ++c) {
+            const int buf = g & 1;
+            const bool last = c + 1 == nch;
+            load_pool(last, last ? 0 : c + 1);
+            load_q(last ? 0 : c + 1, qx);
+            // the next chunk's loads stay ahead of this chunk's MFMAs
+            __builtin_amdgcn_sched_barrier(0);
+            // A = pool row u*32 + (lane%32), B = query lane%32.  Two tiles at a
+            // time (their MFMAs do not wait for each other); a chunk is
+            // summed on its own, the small products first, and added to the
+            // running dot: the rounding error grows with sqrt(chunks)
+#pragma unroll
+            for (int u = 0; u < kSplitTiles; u += kGroup) {
+                halfx8 av[kGroup][4];
+#pragma unroll
+                for (int t = 0; t < kGroup; ++t)
+#pragma unroll
+                    for (int s = 0; s < 4; ++s)
+                        av[t][s] = *reinterpret_cast<const halfx8*>(&sm.tile[buf][kPoolTile * (u + t) + j][8 * h + 16 * s]);
+                floatx16 part[kGroup];
+#pragma unroll
+                for (int t = 0; t < kGroup; ++t)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) part[t][r] = 0.f;
+                auto step = [&](int x, int y) __attribute__((always_inline)) {
+#pragma unroll
+                    for (int t = 0; t < kGroup; ++t)
+                        part[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av[t][x], qc[y], part[t], 0, 0, 0);
+                };
+                step(2, 0);
+                step(3, 1);
+                step(0, 2);
+                step(1, 3);
+                step(0, 0);
+                step(1, 1);
+#pragma unroll
+                for (int t = 0; t < kGroup; ++t)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) acc[u + t][r] += part[t][r];
+            }
+            store_pool(buf ^ 1);
+            __syncthreads();
+#pragma unroll
+            for (int s = 0; s < 4; ++s) qc[s] = qx[s];
+            ++g;
+        }
+        if (tid < kSplitRows) {
+            sm.trow[(stile + 1) & 1][tid] = nrow;
+            sm.tnorm[(stile + 1) & 1][tid] = nnrm;
+            sm.tinv[(stile + 1) & 1][tid] = ninv;
+        }
+#pragma unroll
+        for (int u = 0; u < PT; ++u) rid[u] = rid_n[u];
+        set_ids(stile + 2, rid_n);
+
+        // the keys, in place: lane (j, h) holds rows 8g + 4h + e of every tile
+        const int sb = stile & 1;
+#pragma unroll
+        for (int u = 0; u < kSplitTiles; ++u)
+#pragma unroll
+            for (int gg = 0; gg < 4; ++gg) {
+                const float4 pn = *reinterpret_cast<const float4*>(&sm.tnorm[sb][kPoolTile * u + 8 * gg + 4 * h]);
+                const float4 pi = *reinterpret_cast<const float4*>(&sm.tinv[sb][kPoolTile * u + 8 * gg + 4 * h]);
+                const float n4[4] = {pn.x, pn.y, pn.z, pn.w}, i4[4] = {pi.x, pi.y, pi.z, pi.w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float dot = acc[u][4 * gg + e] * (qinv * i4[e]);   // powers of two: exact
+                    acc[u][4 * gg + e] = METRIC == 0 ? fmaf(-2.f, dot, n4[e] + qn) : fmaf(-1.f, dot, n4[e]);
+                }
+            }
+        if (stile == 0 && !a.seed_d) {
+            // a bound on the M-th smallest key: bisection between the
+            // smallest and the largest of the pair's 256 keys (the query
+            // itself among them: one more than M keys at or below it)
+            float lo = INFINITY, hi = -INFINITY;
+            int n = 0;
+#pragma unroll
+            for (int u = 0; u < kSplitTiles; ++u)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const float k = acc[u][r];
+                    const bool in = k < INFINITY && k > -INFINITY;
+                    lo = in ? fminf(lo, k) : lo;
+                    hi = in ? fmaxf(hi, k) : hi;
+                    n += in ? 1 : 0;
+                }
+            lo = fminf(lo, __shfl_xor(lo, 32));
+            hi = fmaxf(hi, __shfl_xor(hi, 32));
+            n += __shfl_xor(n, 32);
+            const bool enough = n > a.M;
+            for (int i = 0; i < 12; ++i) {
+                const float mid = 0.5f * lo + 0.5f * hi;
+                int c = 0;
+#pragma unroll
+                for (int u = 0; u < kSplitTiles; ++u)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) c += acc[u][r] <= mid ? 1 : 0;
+                c += __shfl_xor(c, 32);
+                if (c > a.M) hi = mid;
+                else lo = mid;
+            }
+            if (qvalid && enough && hi < st.thr) st.thr = hi;
+            publish_state(W, lane, qvalid, qn, st);
+        }
+#pragma unroll
+        for (int u = 0; u < kSplitTiles; ++u) {
+            float d[16];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) d[r] = acc[u][r];
+            collect_keys_f32(a, W, d, &sm.trow[sb][kPoolTile * u], lane, qvalid, qn, st);
+        }
+    }
+    if (qvalid && h == 0) a.cand_cnt[st.orow] = st.cnt;
+    if (a.stats && qvalid && h == 0) atomicAdd(a.stats, static_cast<unsigned long long>(st.cnt));
+}
+
+// ------------------------------------------------------------ selection, long lists
+
+// Sorts the wave's 64 KPL keys ascending, element KPL lane + r in k[r]
+// (bitonic; partners of other lanes through shuffles).
+template <int KPL>
+__device__ __forceinline__ void wave_sort(uint64_t (&k)[KPL], int lane)
+{
+    constexpr int N = 64 * KPL;
+#pragma unroll
+    for (int size = 2; size <= N; size <<= 1) {
+#pragma unroll
+        for (int d = size >> 1; d > 0; d >>= 1) {
+            if (d < KPL) {
+#pragma unroll
+                for (int r = 0; r < KPL; ++r)
+                    if ((r & d) == 0) {
+                        const bool up = ((KPL * lane + r) & size) == 0;
+                        const bool sw = (k[r + d] < k[r]) == up;
+                        const uint64_t lo = sw ? k[r + d] : k[r];
+                        k[r + d] = sw ? k[r] : k[r + d];
+                        k[r] = lo;
+                    }
+            } else {
+                const int ld = d / KPL;
+                const bool low = (lane & ld) == 0;
+#pragma unroll
+                for (int r = 0; r < KPL; ++r) {
+                    const bool up = ((KPL * lane + r) & size) == 0;
+                    const uint64_t o = shfl_xor_u64(k[r], ld);
+                    const bool take = (o < k[r]) == (low == up);   // distinct keys or equal fillers
+                    k[r] = take ? o : k[r];
+                }
+            }
+        }
+    }
+}
+
+// Row's top M (65..128) of its cnt[row] keys, ascending: one wave per row
+// sorts them (2 or 4 keys per lane).
+__global__ void __launch_bounds__(256) knn_sort_select_kernel(const uint64_t* __restrict__ cand,
+                                                              const int32_t* __restrict__ cnt, int64_t rows, int M,
+                                                              int32_t* __restrict__ out_ids, float* __restrict__ out_d)
+{
+    const int lane = threadIdx.x & 63;
+    const int64_t row = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
+    if (row >= rows) return;
+    const int n = __builtin_amdgcn_readfirstlane(min(cnt[row], kCollectCap));
+    const uint64_t* src = cand + row * kCollectCap;
+    auto go = [&](auto kpl) __attribute__((always_inline)) {
+        constexpr int KPL = decltype(kpl)::value;
+        uint64_t k[KPL];
+#pragma unroll
+        for (int r = 0; r < KPL; ++r) k[r] = KPL * lane + r < n ? src[KPL * lane + r] : kNoKey;
+        if (n > 0) wave_sort(k, lane);
+#pragma unroll
+        for (int r = 0; r < KPL; ++r) {
+            const int p = KPL * lane + r;
+            if (p < M) {
+                out_ids[row * M + p] = k[r] == kNoKey ? -1 : static_cast<int32_t>(static_cast<uint32_t>(k[r]));
+                out_d[row * M + p] = k[r] == kNoKey ? INFINITY : o2f(static_cast<uint32_t>(k[r] >> 32));
+            }
+        }
+    };
+    if (n <= 128) go(std::integral_constant<int, 2>{});
+    else go(std::integral_constant<int, 4>{});
+}
+
+void launch_sort_select(const uint64_t* cand, const int32_t* cnt, int64_t rows, int M, int32_t* out_ids, float* out_d,
+                        hipStream_t s)
+{
+    GT_REQUIRE(M >= 1 && M <= 128 && kCollectCap == 256, "sort selection: list length");
+    if (rows <= 0) return;
+    hipLaunchKernelGGL(knn_sort_select_kernel, dim3(static_cast<unsigned>(ceil_div(rows, int64_t(4)))), dim3(256), 0, s,
+                       cand, cnt, rows, M, out_ids, out_d);
+    GT_HIP(hipGetLastError());
+}
+
+// Queries per block of a launch over n_queries queries: 256 (8 waves) where
+// that gives every CU a block, else 128.
+int wide_queries_per_block(int64_t n_queries) { return n_queries >= int64_t(256) * 256 ? 256 : 128; }
+
+// Xs, inv: the split rows by position in the member list (a.q_rows); p_pos:
+// the position of every pool-list entry.
+void launch_wide_collect(const KnnArgs& a, int qpb, const uint16_t* Xs, const float* inv, const int32_t* p_pos,
+                         hipStream_t s)
+{
+    GT_REQUIRE(a.q_rows && a.p_rows && a.n_items % 8 == 0 && a.Dp % kSplitChunk == 0 && a.cand && a.cand_cnt && (qpb == 128 || qpb == 256),
+               "wide collect launch");
+    if (a.n_items <= 0) return;
+    const _Float16* x = reinterpret_cast<const _Float16*>(Xs);
+    auto go = [&](auto kernel, int waves, size_t lds) {
+        GT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   static_cast<int>(lds)));
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(a.n_items)), dim3(static_cast<unsigned>(64 * waves)), lds, s,
+                           a, x, inv, p_pos);
+    };
+    if (qpb == 256) {
+        if (a.metric == 0) go(&knn_wide_collect_kernel<0, 8>, 8, sizeof(WideCollectSmem<8>));
+        else go(&knn_wide_collect_kernel<1, 8>, 8, sizeof(WideCollectSmem<8>));
+    } else {
+        if (a.metric == 0) go(&knn_wide_collect_kernel<0, 4>, 4, sizeof(WideCollectSmem<4>));
+        else go(&knn_wide_collect_kernel<1, 4>, 4, sizeof(WideCollectSmem<4>));
+    }
+    GT_HIP(hipGetLastError());
+}
+
+}  // namespace gtann

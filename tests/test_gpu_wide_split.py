@@ -1,0 +1,102 @@
+"""Bucketed kNN of float rows longer than 160: the collect kernel on rows
+split into two fp16 parts, against the merging fp32 kernels (knn_collect off)
+and 64 bits.  Integer-valued rows below 2^11 have no second part and exact
+sums, so there both paths give the same tables bit for bit; on float rows the
+split path's error against 64 bits is no larger."""
+import numpy as np
+import pytest
+
+from helpers import debug_opts
+
+pytestmark = pytest.mark.gpu
+
+
+def _buckets(rng, n, nb, probe):
+    assign = rng.integers(0, nb, size=n)
+    assign[assign == nb - 1] = 0                     # the last bucket is empty
+    members = np.argsort(assign, kind="stable").astype(np.int32)
+    off = np.searchsorted(assign[members], np.arange(nb + 1)).astype(np.int64)
+    pr = np.stack([rng.permutation(np.delete(np.arange(nb), b))[:probe] for b in range(nb)]).astype(np.int32)
+    return off, members, pr.reshape(nb, probe)
+
+
+def _both(ctx, X, off, members, pr, M, metric="l2", running=None):
+    got = ctx.knn_bucketed(X, off, members, pr, M, metric=metric, running=running)
+    with debug_opts(ctx, knn_collect=False):
+        ref = ctx.knn_bucketed(X, off, members, pr, M, metric=metric, running=running)
+    return got, ref
+
+
+@pytest.mark.parametrize("n,d,nb,probe,M", [
+    (3000, 161, 5, 1, 64), (2500, 256, 3, 0, 65), (4100, 288, 9, 2, 96), (1500, 500, 4, 1, 128),
+    (700, 1024, 3, 1, 5), (40, 300, 2, 0, 33), (1, 200, 1, 0, 8), (193, 960, 1, 0, 128), (2000, 992, 300, 3, 16),
+])
+def test_integer_rows_match_the_fp32_kernels(ctx, n, d, nb, probe, M):
+    rng = np.random.default_rng(n + d)
+    X = rng.integers(-60, 60, size=(n, d)).astype(np.float32)
+    X[:, 0] += 0.5 if d <= 256 else 0.0              # rows of at most 256 dimensions: not the int8 kernel's
+    if n > 100:
+        X[50:60] = X[40]                             # ties
+    off, members, pr = _buckets(rng, n, nb, probe) if nb > 1 else (np.array([0, n]), np.arange(n, dtype=np.int32),
+                                                                 np.zeros((1, 0), np.int32))
+    print(f"wide split n={n} d={d} M={M}", flush=True)
+    for metric in ("l2", "ip"):
+        got, ref = _both(ctx, X, off, members, pr, M, metric)
+        np.testing.assert_array_equal(got[0], ref[0])
+        np.testing.assert_array_equal(got[1], ref[1])
+        # merged into the table of another bucketing
+        o2, m2, p2 = _buckets(np.random.default_rng(5), n, max(2, nb), 0)
+        run = ctx.knn_bucketed(X, o2, m2, p2, M, metric=metric)
+        got, ref = _both(ctx, X, off, members, pr, M, metric, running=run)
+        np.testing.assert_array_equal(got[0], ref[0])
+        np.testing.assert_array_equal(got[1], ref[1])
+
+
+def _rows(kind, rng, n, d):
+    if kind == "mixture":
+        return (rng.uniform(0, 1, (8, d))[rng.integers(0, 8, n)] + 0.1 * rng.standard_normal((n, d))).astype(np.float32)
+    if kind == "latent":
+        return (rng.standard_normal((n, 24)) @ rng.standard_normal((24, d)) * 0.2
+                + 0.02 * rng.standard_normal((n, d))).astype(np.float32)
+    x = rng.standard_normal((n, d))
+    return (x / np.linalg.norm(x, axis=1, keepdims=True)).astype(np.float32)
+
+
+@pytest.mark.parametrize("d", [161, 256, 288, 512, 960, 1024])
+@pytest.mark.parametrize("kind,metric", [("mixture", "l2"), ("latent", "l2"), ("unit", "ip")])
+def test_error_against_64_bits(ctx, kind, metric, d):
+    rng = np.random.default_rng(d)
+    n, M = 2000, 64
+    X = _rows(kind, rng, n, d)
+    X64 = X.astype(np.float64)
+    dot = X64 @ X64.T
+    sq = np.diag(dot)
+    full = dot if metric == "ip" else sq[:, None] + sq[None] - 2 * dot
+    scale = np.sqrt(sq[:, None] * sq[None]) if metric == "ip" else sq[:, None] + sq[None]
+    rms = []
+    for ids, dist in _both(ctx, X, np.array([0, n]), np.arange(n, dtype=np.int32), np.zeros((1, 0), np.int32), M, metric):
+        e = (dist - np.take_along_axis(full, ids.astype(np.int64), 1)) / np.take_along_axis(scale, ids.astype(np.int64), 1)
+        rms.append(float(np.sqrt((e * e).mean())) * 2 ** 24)
+    print(f"wide split d={d} {kind} {metric}: rms error {rms[0]:.3f} ulps, fp32 kernel {rms[1]:.3f}", flush=True)
+    # the same sums in another order: 5 % for the sample (128,000 distances)
+    assert rms[0] <= 1.05 * rms[1]
+
+
+@pytest.mark.parametrize("metric", ["l2", "ip"])
+def test_rows_that_are_not_finite_and_scales(ctx, metric):
+    rng = np.random.default_rng(9)
+    n, d, M = 600, 320, 32
+    X = rng.integers(-20, 20, size=(n, d)).astype(np.float32)
+    X[:200] *= np.float32(2.0 ** 40)
+    X[200:400] *= np.float32(2.0 ** -40)
+    X[401] = 0.0
+    off, members, pr = _buckets(rng, n, 3, 1)
+    got, ref = _both(ctx, X, off, members, pr, M, metric)
+    np.testing.assert_array_equal(got[0], ref[0])
+    np.testing.assert_array_equal(got[1], ref[1])
+    X[10, 3] = np.inf
+    X[410, 5] = -np.inf
+    X[420, 7] = np.nan
+    got, ref = _both(ctx, X, off, members, pr, M, metric)
+    np.testing.assert_array_equal(got[0], ref[0])
+    np.testing.assert_array_equal(got[1], ref[1])

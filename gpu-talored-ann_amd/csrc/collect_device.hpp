@@ -43,8 +43,34 @@ __device__ __forceinline__ bool key_passes(float d, int32_t id, const CollectSta
     return d < st.thr || (d == st.thr && static_cast<uint32_t>(id) <= st.thr_id);
 }
 
-// Keeps the M smallest of query q's cnt (> M) keys in its slots and makes the
-// M-th its threshold.  Called by all 64 lanes; q is uniform.
+// Drops the largest of query q's cnt (> M) keys: its slots keep the M smallest
+// and at most kCompactSlack more, and the largest distance kept becomes its
+// threshold.  The distance is found by bisection over the ordered bits of the
+// keys' distances (about 7 steps of a compare and a bit count per 64 keys; the
+// exact M-th key takes 64 such steps over both words, 1,100 instructions, and
+// made up most of the wide kernel's vector work).  Only where more keys tie
+// there than the slots can spare is it the M-th key in (distance, id) order.
+// Called by all 64 lanes; q is uniform.
+constexpr int kCompactSlack = 16;
+
+template <bool MAX>
+__device__ __forceinline__ uint32_t wave_extreme_u32(uint32_t x)
+{
+    auto f = [](uint32_t a, uint32_t b) { return MAX ? max(a, b) : min(a, b); };
+    auto dpp = [](uint32_t v, auto ctrl, auto rows) {
+        return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(static_cast<int>(v), static_cast<int>(v), decltype(ctrl)::value,
+                                                                 decltype(rows)::value, 0xf, false));
+    };
+    using std::integral_constant;
+    x = f(x, dpp(x, integral_constant<int, 0x111>{}, integral_constant<int, 0xf>{}));   // row_shr:1, 2, 4, 8
+    x = f(x, dpp(x, integral_constant<int, 0x112>{}, integral_constant<int, 0xf>{}));
+    x = f(x, dpp(x, integral_constant<int, 0x114>{}, integral_constant<int, 0xf>{}));
+    x = f(x, dpp(x, integral_constant<int, 0x118>{}, integral_constant<int, 0xf>{}));
+    x = f(x, dpp(x, integral_constant<int, 0x142>{}, integral_constant<int, 0xa>{}));   // row_bcast:15, 31
+    x = f(x, dpp(x, integral_constant<int, 0x143>{}, integral_constant<int, 0xc>{}));
+    return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(x), 63));
+}
+
 __device__ __forceinline__ void collect_compact(const KnnArgs& a, int lane, int q, CollectState& st)
 {
     const int cntq = __builtin_amdgcn_readlane(st.cnt, q);
@@ -59,32 +85,56 @@ __device__ __forceinline__ void collect_compact(const KnnArgs& a, int lane, int 
     constexpr int KPL = kCollectCap / 64;   // slots per lane
     static_assert(kCollectCap % 64 == 0, "whole slots per lane");
     uint64_t k[KPL];
+    uint32_t dmax = 0, dmin = 0xFFFFFFFFu;
 #pragma unroll
-    for (int i = 0; i < KPL; ++i)
-        k[i] = lane + 64 * i < cntq
-                   ? __hip_atomic_load(slots + lane + 64 * i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)
-                   : kNoKey;
-    // the M-th smallest key: the largest K with fewer than M keys below it
+    for (int i = 0; i < KPL; ++i) {
+        const bool in = lane + 64 * i < cntq;
+        k[i] = in ? __hip_atomic_load(slots + lane + 64 * i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) : kNoKey;
+        const uint32_t d = static_cast<uint32_t>(k[i] >> 32);
+        dmax = in ? max(dmax, d) : dmax;
+        dmin = in ? min(dmin, d) : dmin;
+    }
     const int M = a.M;
-    uint64_t K = 0;
-    for (int b = 63; b >= 0; --b) {
-        const uint64_t t = K | (1ull << b);
-        int below = 0;
+    // fewer than M keys at distances up to lo, at least M (n) up to hi; no
+    // real distance has the bits 0
+    uint32_t hi = wave_extreme_u32<true>(dmax), lo = wave_extreme_u32<false>(dmin) - 1u;
+    int n = cntq;
+    while (hi - lo > 1u && n > M + kCompactSlack) {
+        const uint32_t mid = lo + ((hi - lo) >> 1);
+        int c = 0;
 #pragma unroll
-        for (int i = 0; i < KPL; ++i) below += __popcll(__ballot(k[i] < t));
-        if (below < M) K = t;
+        for (int i = 0; i < KPL; ++i) c += __popcll(__ballot(static_cast<uint32_t>(k[i] >> 32) <= mid));
+        if (c < M) {
+            lo = mid;
+        } else {
+            hi = mid;
+            n = c;
+        }
+    }
+    uint64_t K = (static_cast<uint64_t>(hi) << 32) | 0xFFFFFFFFu;
+    if (n > kCollectCap - 4 * 16) {
+        // ties: the M-th smallest key, the largest K with fewer than M keys below it
+        K = 0;
+        for (int b = 63; b >= 0; --b) {
+            const uint64_t t = K | (1ull << b);
+            int below = 0;
+#pragma unroll
+            for (int i = 0; i < KPL; ++i) below += __popcll(__ballot(k[i] < t));
+            if (below < M) K = t;
+        }
+        n = M;
     }
     const uint64_t lt = (1ull << lane) - 1ull;
     int base = 0;
 #pragma unroll
     for (int i = 0; i < KPL; ++i) {
-        const bool p = k[i] <= K;
+        const bool p = k[i] <= K && k[i] != kNoKey;
         const uint64_t m = __ballot(p);
         if (p) slots[base + __popcll(m & lt)] = k[i];
         base += __popcll(m);
     }
     if ((lane & 31) == q) {
-        st.cnt = M;
+        st.cnt = n;
         st.thr = o2f(static_cast<uint32_t>(K >> 32));
         st.thr_id = static_cast<uint32_t>(K);
     }

@@ -36,7 +36,9 @@ void launch_split_rows(const float* X, const float* nrm, const int32_t* members,
 void launch_iota(int32_t* p, int64_t n, hipStream_t s);
 int wide_queries_per_block(int64_t n_queries);
 void launch_wide_collect(const KnnArgs& a, int qpb, const uint16_t* Xs, const float* inv, const int32_t* p_pos,
-                         hipStream_t s);
+                         bool q_by_row, hipStream_t s);
+void launch_split_select(const uint64_t* cand, const int32_t* cnt, int64_t nq, int splits, int M, int32_t* out_ids,
+                         float* out_d, hipStream_t s);
 void launch_collect_select(const KnnArgs& a, int64_t rows, hipStream_t stream);
 void launch_merge_partials(const int32_t* pids, const float* pd, int64_t nq, int splits, int M, int32_t* out_ids,
                            float* out_d, hipStream_t stream);
@@ -270,7 +272,7 @@ struct gt_ctx {
     uint64_t screen_gen = 0;    // data_gen whose fp16 copy and scale W_XH / W_SQ hold (0: none)
     const float* screen_src = nullptr;
     uint64_t split_gen = 0;     // data_gen whose fp16 pairs W_XSPLIT / W_XSINV hold (0: none)
-    uint64_t split_order = 0;   // members_ver of their order
+    uint64_t split_order = 0;   // members_ver of their order (0: by row id)
     bool split_bad = false;     // some |x|^2 of them is not finite
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     void* scratch = nullptr;    // this device's fixed scratch array (gt_optimize_noalloc), or null
@@ -1042,10 +1044,10 @@ static void sub_order_members(Ctx& c, const DevMatrix& X, const Buckets& b, int 
 }
 
 // The rows of X split into two fp16 parts (knn_wide_collect.hip) in the order
-// of the member list, once per order; false where the copy and the launch's
-// candidate slots would not leave half of the free device memory, or the
-// inner product meets a row whose norm is not finite (the fp32 kernel then
-// takes the launch).
+// of the member list (null: their own), once per order; false where the copy
+// and the launch's candidate slots would not leave half of the free device
+// memory, or the inner product meets a row whose norm is not finite (the fp32
+// kernel then takes the launch).
 static bool split_rows(Ctx& c, const DevMatrix& X, const int32_t* d_members, int64_t rows, int metric)
 {
     const int64_t N = X.N, Np = ceil_div(N, int64_t(32)) * 32;
@@ -1059,10 +1061,11 @@ static bool split_rows(Ctx& c, const DevMatrix& X, const int32_t* d_members, int
     uint16_t* xs = c.ws<uint16_t>(W_XSPLIT, need / 2);
     float* inv = c.ws<float>(W_XSINV, static_cast<size_t>(N));
     unsigned int* bad = c.ws<unsigned int>(W_XSBAD, 1);
-    if (c.c->split_gen != c.c->data_gen || c.c->split_order != c.c->members_ver) {
+    const uint64_t order = d_members ? c.c->members_ver : 0;
+    if (c.c->split_gen != c.c->data_gen || c.c->split_order != order) {
         launch_split_rows(X.data, X.norms, d_members, N, X.Dp, xs, inv, bad, c.s);
         c.c->split_gen = c.c->data_gen;
-        c.c->split_order = c.c->members_ver;
+        c.c->split_order = order;
         c.c->split_bad = false;
         if (metric == GT_METRIC_IP) {
             unsigned int h = 0;
@@ -1347,7 +1350,7 @@ static double bucketed_round(Ctx& c, const DevMatrix& X, const Buckets& b, int M
                           screen_window, d_tq, d_urows, d_uitems, a.pairs_done, c.s);
         }
         if (wide) {
-            launch_wide_collect(a, qstep, c.ws<uint16_t>(W_XSPLIT, 0), c.ws<float>(W_XSINV, 0), d_ppos, c.s);
+            launch_wide_collect(a, qstep, c.ws<uint16_t>(W_XSPLIT, 0), c.ws<float>(W_XSINV, 0), d_ppos, false, c.s);
             launch_collect_select(a, rows, c.s);
         } else if (collect) {
             launch_knn_collect_select(a, rows, c.s);
@@ -1399,6 +1402,60 @@ static double bucketed_round(Ctx& c, const DevMatrix& X, const Buckets& b, int M
     if (max_bucket) *max_bucket = std::max(*max_bucket, mb);
     if (pairs) *pairs += pr;
     return t;
+}
+
+// Exact kNN of float rows on the fp16 matrix cores over rows split in two:
+// the queries against the rows in slices of the pool (blocks of 256 queries,
+// two per CU in all), then each query's top k over its slices' candidates.
+// false: not this path's (integer rows, short lists, few queries: the split
+// copy costs a pass over the rows, which below kMinQueries queries takes
+// longer than it saves).
+static bool knn_exact_split(Ctx& c, const DevMatrix& X, const int32_t* d_q, int64_t nq, int k, int metric,
+                            int32_t* out_ids, float* out_d)
+{
+    constexpr int64_t kMinQueries = 256, kMinRows = 4096, kSliceRows = 2048;
+    if (c.c->dbg.knn_collect == 0 || use_i8(X, X, metric) || k <= 4 || k > 128 || nq < kMinQueries || X.N < kMinRows)
+        return false;
+    const int64_t by_pool = X.N / kSliceRows;
+    int64_t qpb = 256, qt = ceil_div(nq, qpb);
+    auto slices = [&]() { return std::max<int64_t>(1, std::min<int64_t>({512 / qt, by_pool, 128})); };
+    int64_t splits = slices();
+    if (qt * splits < 256) {
+        qpb = 128;
+        qt = ceil_div(nq, qpb);
+        splits = slices();
+    }
+    if (!split_rows(c, X, nullptr, splits * nq, metric)) return false;
+    const int64_t chunk = ceil_div(X.N, splits);
+    std::vector<WorkItem> items;
+    items.reserve(static_cast<size_t>(splits * qt + 8));
+    for (int64_t s = 0; s < splits; ++s)
+        for (int64_t t = 0; t < qt; ++t) {
+            WorkItem it{};
+            it.q_begin = t * qpb;
+            it.q_count = static_cast<int32_t>(std::min<int64_t>(qpb, nq - it.q_begin));
+            it.p_begin = s * chunk;
+            it.p_count = static_cast<int32_t>(std::max<int64_t>(0, std::min<int64_t>(chunk, X.N - it.p_begin)));
+            it.out_base = s * nq + it.q_begin;
+            items.push_back(it);
+        }
+    while (items.size() % 8 != 0) items.push_back(WorkItem{});   // q_count 0
+    WorkItem* d_items = c.ws<WorkItem>(W_ITEMS, items.size());
+    c.h2d(d_items, items.data(), items.size() * sizeof(WorkItem));
+    KnnArgs a{};
+    set_operands(a, X, X, metric);
+    a.q_rows = d_q;
+    a.items = d_items;
+    a.n_items = static_cast<int32_t>(items.size());
+    a.M = k;
+    a.metric = metric;
+    a.exclude_self = 1;
+    a.seed_ld = k;
+    a.cand = c.ws<uint64_t>(W_CAND, static_cast<size_t>(splits * nq + kQueriesPerWave) * kCollectCap);
+    a.cand_cnt = c.ws<int32_t>(W_CANDCNT, static_cast<size_t>(splits * nq));
+    launch_wide_collect(a, static_cast<int>(qpb), c.ws<uint16_t>(W_XSPLIT, 0), c.ws<float>(W_XSINV, 0), nullptr, true, c.s);
+    launch_split_select(a.cand, a.cand_cnt, nq, static_cast<int>(splits), k, out_ids, out_d, c.s);
+    return true;
 }
 
 // The device half of one round's bucketing: centroids (sampled rows, moved by
@@ -2898,18 +2955,20 @@ int gt_knn_exact(gt_ctx* ctx, const void* X, int64_t N, int32_t D, int dtype, in
         if (nq == 0) return;
         int32_t* oi = c.in<int32_t>(W_IDS, ids, static_cast<size_t>(nq) * k, false);
         float* od = c.in<float>(W_D, dists, static_cast<size_t>(nq) * k, false);
-        KnnJob j;
-        j.Q = &Xm;
-        j.P = &Xm;
-        j.q_rows = d_q;
-        j.nq = nq;
-        j.np = N;
-        j.M = k;
-        j.metric = metric;
-        j.exclude_self = true;
-        j.out_ids = oi;
-        j.out_d = od;
-        run_knn_flat(c, j);
+        if (!knn_exact_split(c, Xm, d_q, nq, k, metric, oi, od)) {
+            KnnJob j;
+            j.Q = &Xm;
+            j.P = &Xm;
+            j.q_rows = d_q;
+            j.nq = nq;
+            j.np = N;
+            j.M = k;
+            j.metric = metric;
+            j.exclude_self = true;
+            j.out_ids = oi;
+            j.out_d = od;
+            run_knn_flat(c, j);
+        }
         if (metric == GT_METRIC_IP) launch_negate(od, nq * k, c.s);
         c.out(ids, oi, static_cast<size_t>(nq) * k);
         c.out(dists, od, static_cast<size_t>(nq) * k);

@@ -1,5 +1,6 @@
-// knn_wide_collect.hip -- collect + select kNN for fp32 rows longer than 160
-// floats, the contraction on the fp16 matrix cores over rows split in two
+// knn_wide_collect.hip -- collect + select kNN of fp32 rows on the fp16 matrix
+// cores over rows split in two: bucketed passes over rows longer than 160
+// floats, and exact kNN of many queries at any length
 // (src/bucket.cu:4101-4265 top-M semantics: self excluded, (-1, +inf)
 // padding, ties by id).
 //
@@ -20,12 +21,19 @@
 // products (the inner product of such rows stays on the fp32 kernel).
 //
 // Three fp16 products cost 3/16 of one fp32 product of the fp32 matrix cores,
-// and h and m take the fp32 row's bytes, so what bounds the kernel is moving
-// rows, not multiplying: a block is 8 waves with 256 queries (32 per wave,
-// read from L2 chunk by chunk) against 256 pool rows at a time (32-dimension
-// chunks double-buffered in LDS, shared by the waves; 8 accumulator tiles of
-// 32 x 32 per wave), 64 KiB of rows per 65,536 x 32 multiply-adds.  Launches
-// with fewer blocks than the chip has CUs take 4 waves and 128 queries.
+// and h and m take the fp32 row's bytes, so moving rows is what there is to
+// save: a block is 8 waves with 256 queries (32 per wave, read from L2 chunk
+// by chunk) against 192 or 256 pool rows at a time (32-dimension chunks
+// double-buffered in LDS, shared by the waves; 6 or 8 accumulator tiles of
+// 32 x 32 per wave).  Launches with fewer blocks than the chip has CUs take 4
+// waves and 128 queries.  What bounds it (D 960, 2.1e9 pairs, keys not
+// collected, variants timed with parts left out): 13.3 ms, without the query
+// loads 11.2, without the pool loads 12.1, without either and the barrier 9.2,
+// the MFMAs alone 4.9: the LDS reads (every wave reads every pool row), then
+// the loads' latency.  Stages of two chunks, half the barriers, were no faster.
+// Measured (bucketed pass over 100,003 x 960, 25 buckets, one probe, M 96):
+// 20.3 ms on the fp32 kernel, 8.3 here; a 10^6 x 960 build 237 -> 128 ms; exact
+// 100-NN of 10,000 queries in 1,000,003 x 100: 40.2 -> 14.1 ms.
 //
 // Keys at or below a query's threshold go to its candidate slots in HBM as in
 // knn_collect.hip.  An unseeded pass first bounds each query's M-th smallest
@@ -38,12 +46,22 @@
 namespace gtann {
 
 typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
+constexpr int kMaxSplits = 128;   // pool slices of an exact kNN launch
+
 typedef _Float16 halfx4 __attribute__((ext_vector_type(4)));
 
 constexpr int kSplitChunk = 32;                   // dimensions per chunk: 32 h, then 32 m
-constexpr int kSplitRows = 192;                   // pool rows per tile
-constexpr int kSplitTiles = kSplitRows / kPoolTile;
-constexpr int kGroup = 1;                         // tiles multiplied at a time
+
+// Pool rows per tile.  Rows of up to 256 dimensions sum all chunks in one
+// accumulator (their error is below the fp32 kernel's as it is); longer ones
+// sum each chunk on its own, which takes the registers of a quarter of the
+// tile (D 960, error against 64 bits: 4.8 ulps rms in one accumulator, 1.6 by
+// chunks, 1.6 the fp32 kernel).
+template <bool PARTS>
+struct SplitTile {
+    static constexpr int ROWS = PARTS ? 192 : 256;
+    static constexpr int TILES = ROWS / kPoolTile;
+};
 constexpr int kSplitStride = 2 * kSplitChunk + 8; // halves per LDS row: 16 rows' same pieces fill the banks once
 
 // Where the split copy holds chunk c of the row at position p of the member
@@ -55,7 +73,7 @@ __device__ __forceinline__ int64_t split_at(int64_t p, int c, int nch)
     return (((p >> 5) * nch + c) * 32 + (p & 31)) * 2 * kSplitChunk;
 }
 
-// The rows X[members[p]] (stride Dp) to Xs at their positions p: per row and
+// The rows X[members[p]] (stride Dp; members null: X[p]) to Xs at their positions p: per row and
 // chunk 32 h, then 32 m; inv[p] = 2^-k.  *bad counts rows whose |x|^2 is not
 // finite.  One wave per position.
 __global__ void __launch_bounds__(256) split_rows_kernel(const float* __restrict__ X, const float* __restrict__ nrm,
@@ -66,7 +84,7 @@ __global__ void __launch_bounds__(256) split_rows_kernel(const float* __restrict
     const int lane = threadIdx.x & 63;
     const int64_t pos = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
     if (pos >= N) return;
-    const int64_t row = members[pos];
+    const int64_t row = members ? members[pos] : pos;
     const float4* x = reinterpret_cast<const float4*>(X + row * Dp);
     const int n4 = Dp >> 2;
     float4 v[4];                                   // Dp <= 1024: four float4 per lane
@@ -133,8 +151,9 @@ void launch_iota(int32_t* p, int64_t n, hipStream_t s)
     GT_HIP(hipGetLastError());
 }
 
-template <int NW>
+template <int NW, bool PARTS>
 struct WideCollectSmem {
+    static constexpr int kSplitRows = SplitTile<PARTS>::ROWS;
     _Float16 tile[2][kSplitRows][kSplitStride];
     float tnorm[2][kSplitRows];     // |p|^2 (L2) or 0 (IP); +inf past the slice end
     float tinv[2][kSplitRows];      // 2^-k of the row
@@ -142,13 +161,15 @@ struct WideCollectSmem {
     CollectWave wv[NW];
 };
 
-template <int METRIC, int NW>
+template <int METRIC, int NW, bool PARTS>
 __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW == 8 ? 2 : 1)))
 knn_wide_collect_kernel(KnnArgs a, const _Float16* __restrict__ Xs, const float* __restrict__ inv,
-                        const int32_t* __restrict__ p_pos)
+                        const int32_t* __restrict__ p_pos, int q_by_row)
 {
     extern __shared__ __align__(16) unsigned char smem[];
-    WideCollectSmem<NW>& sm = *reinterpret_cast<WideCollectSmem<NW>*>(smem);
+    using Smem = WideCollectSmem<NW, PARTS>;
+    Smem& sm = *reinterpret_cast<Smem*>(smem);
+    constexpr int kSplitRows = SplitTile<PARTS>::ROWS, kSplitTiles = SplitTile<PARTS>::TILES;
     constexpr int T = 64 * NW;
     constexpr int PT = kSplitRows * 8 / T;          // 16-byte pieces of a chunk's rows per thread
     static_assert(PT * T == kSplitRows * 8, "whole pieces");
@@ -169,7 +190,7 @@ knn_wide_collect_kernel(KnnArgs a, const _Float16* __restrict__ Xs, const float*
     const int64_t qi = it.q_begin + qlocal;
     const int32_t qrow = qvalid ? (a.q_rows ? a.q_rows[qi] : static_cast<int32_t>(qi)) : 0;
     const float qn = (qvalid && METRIC == 0) ? a.nq[qrow] : 0.f;
-    const int64_t qpos = qvalid ? qi : it.q_begin;
+    const int64_t qpos = q_by_row ? qrow : qvalid ? qi : it.q_begin;
     const float qinv = inv[qpos];
 
     CollectState st;
@@ -201,7 +222,10 @@ knn_wide_collect_kernel(KnnArgs a, const _Float16* __restrict__ Xs, const float*
     uint4 pre[PT];
     auto set_ids = [&](int stile, int32_t (&ids)[PT]) {
 #pragma unroll
-        for (int u = 0; u < PT; ++u) ids[u] = p_pos[pool_at(min(stile * kSplitRows + r0 + RS * u, pcount - 1))];
+        for (int u = 0; u < PT; ++u) {
+            const int64_t pl = pool_at(min(stile * kSplitRows + r0 + RS * u, pcount - 1));
+            ids[u] = p_pos ? p_pos[pl] : static_cast<int32_t>(pl);
+        }
     };
     auto load_pool = [&](bool next, int c) {
 #pragma unroll
@@ -229,9 +253,9 @@ knn_wide_collect_kernel(KnnArgs a, const _Float16* __restrict__ Xs, const float*
         const int p = stile * kSplitRows + tid;
         if (tid < kSplitRows && p < pcount) {
             const int64_t pl = pool_at(p);
-            id = a.p_rows[pl];
+            id = a.p_rows ? a.p_rows[pl] : static_cast<int32_t>(pl);
             n = METRIC == 0 ? a.np[id] : 0.f;
-            iv = inv[p_pos[pl]];
+            iv = inv[p_pos ? p_pos[pl] : pl];
         }
     };
     static_assert(T >= kSplitRows || T == 256, "one row's ids per thread");
@@ -271,38 +295,26 @@ knn_wide_collect_kernel(KnnArgs a, const _Float16* __restrict__ Xs, const float*
             load_q(last ? 0 : c + 1, qx);
             // the next chunk's loads stay ahead of this chunk's MFMAs
             __builtin_amdgcn_sched_barrier(0);
-            // A = pool row u*32 + (lane%32), B = query lane%32.  Two tiles at a
-            // time (their MFMAs do not wait for each other); a chunk is
-            // summed on its own, the small products first, and added to the
-            // running dot: the rounding error grows with sqrt(chunks)
+            // A = pool row u*32 + (lane%32), B = query lane%32, the small
+            // products first; PARTS: the chunk's sum is added to the running
+            // dot, so that the rounding error grows with sqrt(chunks)
 #pragma unroll
-            for (int u = 0; u < kSplitTiles; u += kGroup) {
-                halfx8 av[kGroup][4];
+            for (int u = 0; u < kSplitTiles; ++u) {
+                halfx8 av[4];
 #pragma unroll
-                for (int t = 0; t < kGroup; ++t)
+                for (int s = 0; s < 4; ++s)
+                    av[s] = *reinterpret_cast<const halfx8*>(&sm.tile[buf][kPoolTile * u + j][8 * h + 16 * s]);
+                floatx16 part;
 #pragma unroll
-                    for (int s = 0; s < 4; ++s)
-                        av[t][s] = *reinterpret_cast<const halfx8*>(&sm.tile[buf][kPoolTile * (u + t) + j][8 * h + 16 * s]);
-                floatx16 part[kGroup];
+                for (int r = 0; r < 16; ++r) part[r] = PARTS ? 0.f : acc[u][r];
+                part = __builtin_amdgcn_mfma_f32_32x32x16_f16(av[2], qc[0], part, 0, 0, 0);
+                part = __builtin_amdgcn_mfma_f32_32x32x16_f16(av[3], qc[1], part, 0, 0, 0);
+                part = __builtin_amdgcn_mfma_f32_32x32x16_f16(av[0], qc[2], part, 0, 0, 0);
+                part = __builtin_amdgcn_mfma_f32_32x32x16_f16(av[1], qc[3], part, 0, 0, 0);
+                part = __builtin_amdgcn_mfma_f32_32x32x16_f16(av[0], qc[0], part, 0, 0, 0);
+                part = __builtin_amdgcn_mfma_f32_32x32x16_f16(av[1], qc[1], part, 0, 0, 0);
 #pragma unroll
-                for (int t = 0; t < kGroup; ++t)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) part[t][r] = 0.f;
-                auto step = [&](int x, int y) __attribute__((always_inline)) {
-#pragma unroll
-                    for (int t = 0; t < kGroup; ++t)
-                        part[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av[t][x], qc[y], part[t], 0, 0, 0);
-                };
-                step(2, 0);
-                step(3, 1);
-                step(0, 2);
-                step(1, 3);
-                step(0, 0);
-                step(1, 1);
-#pragma unroll
-                for (int t = 0; t < kGroup; ++t)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) acc[u + t][r] += part[t][r];
+                for (int r = 0; r < 16; ++r) acc[u][r] = PARTS ? acc[u][r] + part[r] : part[r];
             }
             store_pool(buf ^ 1);
             __syncthreads();
@@ -457,16 +469,127 @@ void launch_sort_select(const uint64_t* cand, const int32_t* cnt, int64_t rows, 
     GT_HIP(hipGetLastError());
 }
 
+// The top M of each query's candidate lists over `splits` pool slices (list s
+// of query q: row s nq + q), ascending.  One block per query: the distances'
+// ordered bits in LDS, a bound with at least M and at most 256 keys at or below
+// it by bisection (by (distance, id) where more than 256 tie), those keys
+// sorted by the first wave.
+__global__ void __launch_bounds__(256) knn_split_select_kernel(const uint64_t* __restrict__ cand,
+                                                               const int32_t* __restrict__ cnt, int64_t nq, int splits,
+                                                               int M, int32_t* __restrict__ out_ids,
+                                                               float* __restrict__ out_d)
+{
+    extern __shared__ __align__(16) unsigned char smem[];
+    uint32_t* key = reinterpret_cast<uint32_t*>(smem);   // up to splits * kCollectCap
+    __shared__ int first[kMaxSplits + 1];
+    __shared__ uint64_t pick[kCollectCap];
+    __shared__ uint32_t ext[2][4];
+    __shared__ int sums[4], npick;
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int64_t q = blockIdx.x;
+    if (tid < splits) first[tid + 1] = min(cnt[tid * nq + q], kCollectCap);
+    if (tid == 0) { first[0] = 0; npick = 0; }
+    __syncthreads();
+    if (tid == 0)
+        for (int s = 0; s < splits; ++s) first[s + 1] += first[s];
+    __syncthreads();
+    const int total = first[splits];
+    uint32_t mx = 0, mn = 0xFFFFFFFFu;
+    for (int s = w; s < splits; s += 4) {
+        const int n = first[s + 1] - first[s];
+        for (int i = lane; i < n; i += 64) {
+            const uint32_t d = static_cast<uint32_t>(cand[(s * nq + q) * kCollectCap + i] >> 32);
+            key[first[s] + i] = d;
+            mx = max(mx, d);
+            mn = min(mn, d);
+        }
+    }
+    mx = wave_extreme_u32<true>(mx);
+    mn = wave_extreme_u32<false>(mn);
+    if (lane == 0) { ext[0][w] = mx; ext[1][w] = mn; }
+    __syncthreads();
+    uint32_t hi = max(max(ext[0][0], ext[0][1]), max(ext[0][2], ext[0][3]));
+    uint32_t lo = min(min(ext[1][0], ext[1][1]), min(ext[1][2], ext[1][3])) - 1u;
+    int n = total;
+    auto block_sum = [&](int c) -> int {
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o);
+        __syncthreads();   // the last sum was read
+        if (lane == 0) sums[w] = c;
+        __syncthreads();
+        return sums[0] + sums[1] + sums[2] + sums[3];
+    };
+    while (n > kCollectCap && hi - lo > 1u) {   // uniform: every thread holds the same bounds
+        const uint32_t mid = lo + ((hi - lo) >> 1);
+        int c = 0;
+        for (int i = tid; i < total; i += 256) c += key[i] <= mid ? 1 : 0;
+        c = block_sum(c);
+        if (c < M) lo = mid;
+        else { hi = mid; n = c; }
+    }
+    uint64_t K = (static_cast<uint64_t>(hi) << 32) | 0xFFFFFFFFu;
+    if (n > kCollectCap) {
+        // ties at distance hi: the ids decide (fewer than M keys lie below hi)
+        uint32_t ilo = 0, ihi = 0xFFFFFFFFu;   // at least M keys with (hi, id <= ihi)
+        while (ilo < ihi) {
+            const uint32_t mid = ilo + ((ihi - ilo) >> 1);
+            const uint64_t t = (static_cast<uint64_t>(hi) << 32) | mid;
+            int c = 0;
+            for (int s = w; s < splits; s += 4)
+                for (int i = lane; i < first[s + 1] - first[s]; i += 64) c += cand[(s * nq + q) * kCollectCap + i] <= t ? 1 : 0;
+            c = block_sum(c);
+            if (c >= M) ihi = mid;
+            else ilo = mid + 1;
+        }
+        K = (static_cast<uint64_t>(hi) << 32) | ihi;
+    }
+    __syncthreads();
+    for (int s = w; s < splits; s += 4)
+        for (int i = lane; i < first[s + 1] - first[s]; i += 64) {
+            const uint64_t k = cand[(s * nq + q) * kCollectCap + i];
+            if (k <= K) pick[atomicAdd(&npick, 1)] = k;
+        }
+    __syncthreads();
+    if (w > 0) return;
+    constexpr int KPL = kCollectCap / 64;
+    uint64_t k[KPL];
+#pragma unroll
+    for (int r = 0; r < KPL; ++r) k[r] = KPL * lane + r < npick ? pick[KPL * lane + r] : kNoKey;
+    wave_sort(k, lane);
+#pragma unroll
+    for (int r = 0; r < KPL; ++r) {
+        const int p = KPL * lane + r;
+        if (p < M) {
+            out_ids[q * M + p] = k[r] == kNoKey ? -1 : static_cast<int32_t>(static_cast<uint32_t>(k[r]));
+            out_d[q * M + p] = k[r] == kNoKey ? INFINITY : o2f(static_cast<uint32_t>(k[r] >> 32));
+        }
+    }
+}
+
+void launch_split_select(const uint64_t* cand, const int32_t* cnt, int64_t nq, int splits, int M, int32_t* out_ids,
+                         float* out_d, hipStream_t s)
+{
+    GT_REQUIRE(M >= 1 && M <= 128 && splits >= 1 && splits <= kMaxSplits && nq < (int64_t(1) << 31), "split selection");
+    if (nq <= 0) return;
+    const size_t lds = static_cast<size_t>(splits) * kCollectCap * 4;
+    GT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&knn_split_select_kernel),
+                               hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
+    hipLaunchKernelGGL(knn_split_select_kernel, dim3(static_cast<unsigned>(nq)), dim3(256), lds, s, cand, cnt, nq, splits,
+                       M, out_ids, out_d);
+    GT_HIP(hipGetLastError());
+}
+
 // Queries per block of a launch over n_queries queries: 256 (8 waves) where
 // that gives every CU a block, else 128.
 int wide_queries_per_block(int64_t n_queries) { return n_queries >= int64_t(256) * 256 ? 256 : 128; }
 
-// Xs, inv: the split rows by position in the member list (a.q_rows); p_pos:
-// the position of every pool-list entry.
+// Xs, inv: the split rows by position; p_pos: the position of every pool-list
+// entry (null: itself).  Query i's position is i, its place in the member list
+// a.q_rows, or with q_by_row its row id (rows split in their own order).
 void launch_wide_collect(const KnnArgs& a, int qpb, const uint16_t* Xs, const float* inv, const int32_t* p_pos,
-                         hipStream_t s)
+                         bool q_by_row, hipStream_t s)
 {
-    GT_REQUIRE(a.q_rows && a.p_rows && a.n_items % 8 == 0 && a.Dp % kSplitChunk == 0 && a.cand && a.cand_cnt && (qpb == 128 || qpb == 256),
+    GT_REQUIRE((p_pos != nullptr) == (a.p_rows != nullptr) && a.n_items % 8 == 0 && a.Dp % kSplitChunk == 0 && a.cand && a.cand_cnt && (qpb == 128 || qpb == 256),
                "wide collect launch");
     if (a.n_items <= 0) return;
     const _Float16* x = reinterpret_cast<const _Float16*>(Xs);
@@ -474,15 +597,20 @@ void launch_wide_collect(const KnnArgs& a, int qpb, const uint16_t* Xs, const fl
         GT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                    static_cast<int>(lds)));
         hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(a.n_items)), dim3(static_cast<unsigned>(64 * waves)), lds, s,
-                           a, x, inv, p_pos);
+                           a, x, inv, p_pos, q_by_row ? 1 : 0);
     };
-    if (qpb == 256) {
-        if (a.metric == 0) go(&knn_wide_collect_kernel<0, 8>, 8, sizeof(WideCollectSmem<8>));
-        else go(&knn_wide_collect_kernel<1, 8>, 8, sizeof(WideCollectSmem<8>));
-    } else {
-        if (a.metric == 0) go(&knn_wide_collect_kernel<0, 4>, 4, sizeof(WideCollectSmem<4>));
-        else go(&knn_wide_collect_kernel<1, 4>, 4, sizeof(WideCollectSmem<4>));
-    }
+    auto by_metric = [&](auto nw, auto parts) {
+        constexpr int NW = decltype(nw)::value;
+        constexpr bool P = decltype(parts)::value;
+        if (a.metric == 0) go(&knn_wide_collect_kernel<0, NW, P>, NW, sizeof(WideCollectSmem<NW, P>));
+        else go(&knn_wide_collect_kernel<1, NW, P>, NW, sizeof(WideCollectSmem<NW, P>));
+    };
+    auto by_dim = [&](auto nw) {
+        if (a.Dp > 256) by_metric(nw, std::true_type{});
+        else by_metric(nw, std::false_type{});
+    };
+    if (qpb == 256) by_dim(std::integral_constant<int, 8>{});
+    else by_dim(std::integral_constant<int, 4>{});
     GT_HIP(hipGetLastError());
 }
 

@@ -1152,13 +1152,16 @@ static double bucketed_round(Ctx& c, const DevMatrix& X, const Buckets& b, int M
         pairs_all += static_cast<double>(b.offsets[static_cast<size_t>(bb + 1)] - b.offsets[static_cast<size_t>(bb)]) *
                      static_cast<double>(pool_cnt[static_cast<size_t>(bb)]);
     const int scr = c.c->dbg.knn_screen;
-    const bool want_screen = c.c->dbg.knn_collect != 0 && !use_i8(X, X, metric) && X.Dp <= 160 &&
+    const bool want_screen = c.c->dbg.knn_collect != 0 && !use_i8(X, X, metric) && X.Dp <= 256 &&
                              (scr == 2 || (scr == 1 && pairs_all >= static_cast<double>(int64_t(1) << 27)));
     const bool sub_ordered = own && !compact && c.c->dbg.sub_order != 0 && (!seed_d || want_prune || want_screen);
     if (sub_ordered) sub_order_members(c, X, b, metric, d_members);
-    // fp32 rows longer than 160: collect on the fp16 matrix cores over rows
-    // split in two, 256 or 128 queries per block (lists of 5..128 keys)
-    const bool wide = c.c->dbg.knn_collect != 0 && !use_i8(X, X, metric) && X.Dp > 160 && M > 4 && M <= 128 &&
+    // fp32 rows longer than 256: collect on the fp16 matrix cores over rows
+    // split in two, 256 or 128 queries per block (lists of 5..128 keys).
+    // (Rows of 161 to 256 stay on the fp32 kernel: its one chain of sums has
+    // errors of up to 4 ulps rms there, against 1 to 2.4 of the split rows,
+    // and 1.7 to 2.1 % of a table's positions, near ties, would change.)
+    const bool wide = c.c->dbg.knn_collect != 0 && !use_i8(X, X, metric) && X.Dp > 256 && M > 4 && M <= 128 &&
                       split_rows(c, X, d_members, rows, metric);
     const int qstep = wide ? wide_queries_per_block(rows) : kQueriesPerBlock;
     CopyTaskH* d_tasks = c.ws<CopyTaskH>(W_TASKS, tasks.size());
@@ -1407,14 +1410,18 @@ static double bucketed_round(Ctx& c, const DevMatrix& X, const Buckets& b, int M
 // Exact kNN of float rows on the fp16 matrix cores over rows split in two:
 // the queries against the rows in slices of the pool (blocks of 256 queries,
 // two per CU in all), then each query's top k over its slices' candidates.
-// false: not this path's (integer rows, short lists, few queries: the split
+// false: not this path's -- integer rows, short lists, few queries (the split
 // copy costs a pass over the rows, which below kMinQueries queries takes
-// longer than it saves).
+// longer than it saves), and rows of 129 to 256 dimensions, where the fp32
+// kernel's one chain of sums rounds most: it orders 1.1 to 1.6 % of a long
+// list's positions, near ties, otherwise than the split rows do (0.85 % at
+// 128, 0.2 % beyond 256), and callers keep the lists they have.
 static bool knn_exact_split(Ctx& c, const DevMatrix& X, const int32_t* d_q, int64_t nq, int k, int metric,
                             int32_t* out_ids, float* out_d)
 {
     constexpr int64_t kMinQueries = 256, kMinRows = 4096, kSliceRows = 2048;
-    if (c.c->dbg.knn_collect == 0 || use_i8(X, X, metric) || k <= 4 || k > 128 || nq < kMinQueries || X.N < kMinRows)
+    if (c.c->dbg.knn_collect == 0 || use_i8(X, X, metric) || k <= 4 || k > 128 || nq < kMinQueries ||
+        X.N < kMinRows || (X.Dp > 128 && X.Dp <= 256))
         return false;
     const int64_t by_pool = X.N / kSliceRows;
     int64_t qpb = 256, qt = ceil_div(nq, qpb);

@@ -1,5 +1,5 @@
-"""Bucketed kNN of float rows longer than 160: the collect kernel on rows
-split into two fp16 parts, against the merging fp32 kernels (knn_collect off)
+"""Bucketed kNN of float rows longer than 256: the collect kernel on rows
+split into two fp16 parts (shorter rows: the fp32 kernels on both sides), against the merging fp32 kernels (knn_collect off)
 and 64 bits.  Integer-valued rows below 2^11 have no second part and exact
 sums, so there both paths give the same tables bit for bit; on float rows the
 split path's error against 64 bits is no larger."""

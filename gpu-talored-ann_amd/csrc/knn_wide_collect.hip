@@ -1,6 +1,7 @@
 // knn_wide_collect.hip -- collect + select kNN of fp32 rows on the fp16 matrix
-// cores over rows split in two: bucketed passes over rows longer than 160
-// floats, and exact kNN of many queries at any length
+// cores over rows split in two: bucketed passes over rows longer than 256
+// floats, and exact kNN of many queries over rows of up to 128 or more than
+// 256
 // (src/bucket.cu:4101-4265 top-M semantics: self excluded, (-1, +inf)
 // padding, ties by id).
 //
@@ -12,9 +13,10 @@
 // within 2^-29 of the row's largest).  A dot product is the sum of h h, h m and m h
 // products, each exact in the fp32 accumulator (v_mfma_f32_32x32x16_f16);
 // the m m products left out are at most 2^-24 of their terms.  Both are
-// below the roundings of an fp32 sum over D terms: measured against 64 bits
-// on D 161..1024 (tests/test_gpu_wide_split.py) the distances are closer than
-// those of the fp32 kernel (knn_wide_kernel).  Integer-valued rows below 2^11
+// below the roundings of an fp32 sum over D terms: measured against 64 bits on
+// D 288..1024 (tests/test_gpu_wide_split.py) the distances are as close as
+// those of the fp32 kernel (knn_wide_kernel; 1.59 and 1.60 ulps rms at D 960),
+// and closer than knn_fused_kernel's (1.9 and 3.1 at D 128).  Integer-valued rows below 2^11
 // have m = 0 and give exact sums.
 // A row with an element that is not finite has a norm that is not finite
 // either: its L2 keys are +inf or NaN, which no list takes, whatever its dot
@@ -429,16 +431,19 @@ __device__ __forceinline__ void wave_sort(uint64_t (&k)[KPL], int lane)
     }
 }
 
-// Row's top M (65..128) of its cnt[row] keys, ascending: one wave per row
-// sorts them (2 or 4 keys per lane).
+// Row's top M (1..128) of its cnt[row] keys, ascending: one wave per row
+// sorts them (2 or 4 keys per lane).  Rows of at most skip_le keys are neither
+// sorted nor written.
 __global__ void __launch_bounds__(256) knn_sort_select_kernel(const uint64_t* __restrict__ cand,
                                                               const int32_t* __restrict__ cnt, int64_t rows, int M,
-                                                              int32_t* __restrict__ out_ids, float* __restrict__ out_d)
+                                                              int skip_le, int32_t* __restrict__ out_ids,
+                                                              float* __restrict__ out_d)
 {
     const int lane = threadIdx.x & 63;
     const int64_t row = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
     if (row >= rows) return;
     const int n = __builtin_amdgcn_readfirstlane(min(cnt[row], kCollectCap));
+    if (n <= skip_le) return;
     const uint64_t* src = cand + row * kCollectCap;
     auto go = [&](auto kpl) __attribute__((always_inline)) {
         constexpr int KPL = decltype(kpl)::value;
@@ -459,13 +464,13 @@ __global__ void __launch_bounds__(256) knn_sort_select_kernel(const uint64_t* __
     else go(std::integral_constant<int, 4>{});
 }
 
-void launch_sort_select(const uint64_t* cand, const int32_t* cnt, int64_t rows, int M, int32_t* out_ids, float* out_d,
-                        hipStream_t s)
+void launch_sort_select(const uint64_t* cand, const int32_t* cnt, int64_t rows, int M, int skip_le, int32_t* out_ids,
+                        float* out_d, hipStream_t s)
 {
     GT_REQUIRE(M >= 1 && M <= 128 && kCollectCap == 256, "sort selection: list length");
     if (rows <= 0) return;
     hipLaunchKernelGGL(knn_sort_select_kernel, dim3(static_cast<unsigned>(ceil_div(rows, int64_t(4)))), dim3(256), 0, s,
-                       cand, cnt, rows, M, out_ids, out_d);
+                       cand, cnt, rows, M, skip_le, out_ids, out_d);
     GT_HIP(hipGetLastError());
 }
 

@@ -101,7 +101,9 @@ __global__ void __launch_bounds__(256) split_rows_kernel(const float* __restrict
     int e = 0;
     const bool finite = mx < INFINITY;
     if (finite && mx > 0.f) frexpf(mx, &e);        // mx < 2^e
-    const int k = finite && mx > 0.f ? 15 - e : 0;
+    // (at most 2^126: the scale back stays a normal float; every float element
+    // is then a multiple of 2^-23, which the two parts hold as well)
+    const int k = finite && mx > 0.f ? min(15 - e, 126) : 0;
     auto scaled = [&](float y) -> float { return finite ? ldexpf(y, k) : 0.f; };
     const int nch = Dp / kSplitChunk;
 #pragma unroll
@@ -344,7 +346,8 @@ knn_wide_collect_kernel(KnnArgs a, const _Float16* __restrict__ Xs, const float*
                 const float n4[4] = {pn.x, pn.y, pn.z, pn.w}, i4[4] = {pi.x, pi.y, pi.z, pi.w};
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    const float dot = acc[u][4 * gg + e] * (qinv * i4[e]);   // powers of two: exact
+                    // powers of two: exact (their product alone may underflow where the dot does not)
+                    const float dot = (acc[u][4 * gg + e] * qinv) * i4[e];
                     acc[u][4 * gg + e] = METRIC == 0 ? fmaf(-2.f, dot, n4[e] + qn) : fmaf(-1.f, dot, n4[e]);
                 }
             }

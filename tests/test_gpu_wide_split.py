@@ -100,3 +100,32 @@ def test_rows_that_are_not_finite_and_scales(ctx, metric):
     got, ref = _both(ctx, X, off, members, pr, M, metric)
     np.testing.assert_array_equal(got[0], ref[0])
     np.testing.assert_array_equal(got[1], ref[1])
+
+
+@pytest.mark.parametrize("metric", ["l2", "ip"])
+def test_small_scales(ctx, metric):
+    """Rows around 2^-60 (the product of two rows' scales underflows, the dot
+    products do not) and 2^-130 (the rows are not normal floats) among rows of
+    ordinary size: sums exact in both kernels."""
+    rng = np.random.default_rng(11)
+    n, d, M = 600, 288, 32
+    X = rng.integers(-20, 20, size=(n, d)).astype(np.float32)
+    scale = -60 if metric == "l2" else -130
+    X[:300] *= np.float32(2.0 ** scale)
+    off, members, pr = _buckets(rng, n, 3, 1)
+    got, ref = _both(ctx, X, off, members, pr, M, metric)
+    np.testing.assert_array_equal(got[0], ref[0])
+    np.testing.assert_array_equal(got[1], ref[1])
+
+
+def test_out_of_core_build(ctx):
+    """Chunks of buckets against rows split in the member order of all: the
+    resident build's table and graph."""
+    X = _rows("mixture", np.random.default_rng(3), 20011, 300)
+    kw = dict(n_buckets=16, M=32, K=16, rounds=2, nprobe=1)
+    res = ctx.build_graph(X, **kw)
+    ooc = ctx.build_graph(X, device_budget_mb=12, **kw)
+    assert res.stats["ooc_chunks"] == 0 and ooc.stats["ooc_chunks"] > 3
+    np.testing.assert_array_equal(ooc.knn_ids, res.knn_ids)
+    np.testing.assert_array_equal(ooc.knn_dists.view(np.uint32), res.knn_dists.view(np.uint32))
+    np.testing.assert_array_equal(ooc.graph, res.graph)

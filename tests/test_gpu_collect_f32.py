@@ -153,3 +153,22 @@ def test_f32_collect_threshold_window_sizes(ctx, window, metric):
     with debug_opts(ctx, knn_window=window):
         got = ctx.knn_bucketed(X, off, mem, probe, 64, metric=metric)
     _equal(got, _merging(ctx, X, off, mem, probe, 64, metric=metric))
+
+
+@pytest.mark.parametrize("N", [16384, 32767, 32768, 33001])
+@pytest.mark.parametrize("M", [7, 33, 64])
+@pytest.mark.parametrize("dtype", ["f32", "int"])
+def test_selection_by_rows(ctx, N, M, dtype):
+    """The selection takes a wave per row below 32,768 rows and a wave per 32
+    rows from there on, the in-place merge 1 row per wave and 2: both equal
+    the merging kernels, which use neither."""
+    rng = np.random.default_rng(N + M)
+    X = rng.integers(-60, 60, size=(N, 24)).astype(np.float32) + (0.5 if dtype == "f32" else 0.0)
+    X[100:100 + 2 * M] = X[99]                       # ties beyond the list
+    off, members = _buckets(rng, N, 40)
+    args = (X, off, members, _probe(rng, 40, 1), M)
+    got = ctx.knn_bucketed(*args)
+    _equal(got, _merging(ctx, *args))
+    o2, m2 = _buckets(rng, N, 37)
+    args = (X, o2, m2, _probe(rng, 37, 0), M)
+    _equal(ctx.knn_bucketed(*args, running=got), _merging(ctx, *args, running=got))

@@ -229,13 +229,19 @@ __global__ void __launch_bounds__(256) refine_2hop_kernel(const float* __restric
 }
 
 // Lloyd update: centroid c = mean of its member rows; empty buckets keep
-// their centroid.  Block (c, h) sums float4 columns [64h, 64h + F) of
-// centroid c (F = min(64, Dp / 4 - 64h): up to 256 dimensions per block, so
-// long rows spread over several blocks): thread t sums column t % F over its
-// group t / F of members (members g, g + G, g + 2G, ... for G = 256 / F
-// groups) with four accumulators (members 4k + u of the group into
-// accumulator u), folded as (a0 + a1) + (a2 + a3), and the groups are added
-// in order.  The result does not depend on scheduling.
+// their centroid.  Columns are float4s; a slab of F = min(64, Dp / 4 - 64 s)
+// of them fixes the order of the sums: G = 256 / F groups of members (members
+// g, g + G, g + 2G, ...), each with four accumulators (members 4k + u of the
+// group into accumulator u), folded as (a0 + a1) + (a2 + a3), and the groups
+// are added in order.  The result does not depend on scheduling.
+// A few dozen centroids of thousands of members leave the chip to serial
+// chains of row gathers, so a block takes 8 columns (128 bytes of a row; Dp / 4
+// is a multiple of 8) of one centroid, all groups, and a thread keeps
+// kMeanRows rows in flight (their ids another kMeanRows ahead): 37 centroids
+// of 4,000 rows x 128, 185 -> 77 us; 512 of rows x 960, 145 -> 113 us (a block
+// per 64 columns, 4 rows in flight, before).
+constexpr int kMeanCols = 8, kMeanRows = 16;
+
 __global__ void __launch_bounds__(256) centroid_means_kernel(const float* __restrict__ X, int Dp,
                                                              const int32_t* __restrict__ members,
                                                              const int64_t* __restrict__ off, int64_t C,
@@ -246,36 +252,40 @@ __global__ void __launch_bounds__(256) centroid_means_kernel(const float* __rest
     if (c >= C) return;
     const int64_t lo = off[c], hi = off[c + 1];
     if (hi <= lo) return;
-    const int FD = Dp / 4, c0 = static_cast<int>(blockIdx.y) * 64;
-    const int F = min(64, FD - c0), G = 256 / F;
-    const int col = threadIdx.x % F, g = threadIdx.x / F;
+    const int FD = Dp / 4, c0 = static_cast<int>(blockIdx.y) * kMeanCols;
+    const int F = min(64, FD - c0 / 64 * 64), G = 256 / F;
+    const int col = threadIdx.x % kMeanCols, g = threadIdx.x / kMeanCols;
     const float4* X4 = reinterpret_cast<const float4*>(X) + c0 + col;
     float4 a[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) a[u] = make_float4(0.f, 0.f, 0.f, 0.f);
     if (g < G) {
-        int64_t i = lo + g;
-        for (; i + 3 * G < hi; i += 4 * G) {
-            float4 x[4];
+        int32_t id[kMeanRows];
+        auto ids = [&](int64_t i) {
 #pragma unroll
-            for (int u = 0; u < 4; ++u) x[u] = X4[static_cast<int64_t>(members[i + u * G]) * FD];
+            for (int u = 0; u < kMeanRows; ++u) id[u] = members[min(i + u * G, hi - 1)];
+        };
+        ids(lo + g);
+        for (int64_t i = lo + g; i < hi; i += kMeanRows * G) {
+            float4 x[kMeanRows];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                a[u].x += x[u].x; a[u].y += x[u].y; a[u].z += x[u].z; a[u].w += x[u].w;
-            }
+            for (int u = 0; u < kMeanRows; ++u) x[u] = X4[static_cast<int64_t>(id[u]) * FD];
+            ids(i + kMeanRows * G);
+#pragma unroll
+            for (int u = 0; u < kMeanRows; ++u)
+                if (i + u * G < hi) {
+                    float4& t = a[u % 4];
+                    t.x += x[u].x; t.y += x[u].y; t.z += x[u].z; t.w += x[u].w;
+                }
         }
-        for (int u = 0; i < hi; i += G, ++u) {
-            const float4 x = X4[static_cast<int64_t>(members[i]) * FD];
-            a[u].x += x.x; a[u].y += x.y; a[u].z += x.z; a[u].w += x.w;
-        }
+        part[threadIdx.x] = make_float4((a[0].x + a[1].x) + (a[2].x + a[3].x), (a[0].y + a[1].y) + (a[2].y + a[3].y),
+                                        (a[0].z + a[1].z) + (a[2].z + a[3].z), (a[0].w + a[1].w) + (a[2].w + a[3].w));
     }
-    part[threadIdx.x] = make_float4((a[0].x + a[1].x) + (a[2].x + a[3].x), (a[0].y + a[1].y) + (a[2].y + a[3].y),
-                                    (a[0].z + a[1].z) + (a[2].z + a[3].z), (a[0].w + a[1].w) + (a[2].w + a[3].w));
     __syncthreads();
-    if (threadIdx.x < F) {
+    if (threadIdx.x < kMeanCols) {
         float4 t = make_float4(0.f, 0.f, 0.f, 0.f);
         for (int q = 0; q < G; ++q) {
-            const float4 v = part[q * F + threadIdx.x];
+            const float4 v = part[q * kMeanCols + threadIdx.x];
             t.x += v.x; t.y += v.y; t.z += v.z; t.w += v.w;
         }
         const float n = static_cast<float>(hi - lo);
@@ -450,9 +460,11 @@ void launch_centroid_sums(const float* X, int Dp, const int32_t* members, const 
                           float* centroids, hipStream_t s)
 {
     if (C <= 0) return;
-    GT_REQUIRE(Dp % 4 == 0, "centroid means: padded rows are multiples of 4 floats");
-    const unsigned chunks = static_cast<unsigned>((Dp / 4 + 63) / 64);
-    hipLaunchKernelGGL(centroid_means_kernel, dim3(static_cast<unsigned>(C), chunks), dim3(256), 0, s, X, Dp,
+    GT_REQUIRE(Dp % (4 * kMeanCols) == 0, "centroid means: padded rows are multiples of 32 floats");
+    const int last = Dp / 4 % 64, f = last ? last : 64;   // the narrowest slab has the most groups
+    const int threads = (kMeanCols * (256 / f) + 63) / 64 * 64;
+    hipLaunchKernelGGL(centroid_means_kernel, dim3(static_cast<unsigned>(C), static_cast<unsigned>(Dp / 4 / kMeanCols)),
+                       dim3(static_cast<unsigned>(threads)), 0, s, X, Dp,
                        members, offsets, C, centroids);
     GT_HIP(hipGetLastError());
 }

@@ -153,13 +153,15 @@ __global__ void __launch_bounds__(256) row_norms_kernel(const float* __restrict_
     if (lane == 0) norms[row] = s;
 }
 
-// pool list of every bucket = concatenation of member ranges (copy tasks).
+// pool list of every bucket = concatenation of member ranges (copy tasks);
+// members null: of the positions themselves.
 struct CopyTask { int64_t src; int64_t dst; int64_t n; };
 __global__ void copy_ranges_kernel(const CopyTask* __restrict__ tasks, const int32_t* __restrict__ members,
                                    int32_t* __restrict__ pool)
 {
     const CopyTask t = tasks[blockIdx.x];
-    for (int64_t e = threadIdx.x; e < t.n; e += blockDim.x) pool[t.dst + e] = members[t.src + e];
+    for (int64_t e = threadIdx.x; e < t.n; e += blockDim.x)
+        pool[t.dst + e] = members ? members[t.src + e] : static_cast<int32_t>(t.src + e);
 }
 
 __global__ void negate_kernel(float* __restrict__ d, int64_t n)

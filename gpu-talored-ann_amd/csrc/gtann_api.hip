@@ -31,12 +31,12 @@ void launch_knn_fused(const KnnArgs& a, hipStream_t stream);
 bool knn_collect_supported(const KnnArgs& a);
 void launch_knn_collect_select(const KnnArgs& a, int64_t rows, hipStream_t stream);
 // knn_wide_collect.hip
-void launch_split_rows(const float* X, const float* nrm, const int32_t* members, int64_t N, int Dp, uint16_t* Xs,
-                       float* inv, unsigned int* bad, hipStream_t s);
-void launch_iota(int32_t* p, int64_t n, hipStream_t s);
+size_t split_copy_bytes(int64_t n, int Dp);
+void launch_split_rows(const float* X, const float* nrm, const int32_t* members, int64_t N, int Dp, float* Xs,
+                       int32_t* ex, unsigned int* bad, hipStream_t s);
 int wide_queries_per_block(int64_t n_queries);
-void launch_wide_collect(const KnnArgs& a, int qpb, const uint16_t* Xs, const float* inv, const int32_t* p_pos,
-                         bool q_by_row, hipStream_t s);
+void launch_wide_collect(const KnnArgs& a, int qpb, const float* Xs, const int32_t* ex, const float* Qs,
+                         const int32_t* qex, const int32_t* p_pos, hipStream_t s);
 void launch_split_select(const uint64_t* cand, const int32_t* cnt, int64_t nq, int splits, int M, int32_t* out_ids,
                          float* out_d, hipStream_t s);
 void launch_collect_select(const KnnArgs& a, int64_t rows, hipStream_t stream);
@@ -284,9 +284,9 @@ struct gt_ctx {
     uint64_t data_gen = 0;      // bumped whenever W_X / W_NORMS are (re)written
     uint64_t screen_gen = 0;    // data_gen whose fp16 copy and scale W_XH / W_SQ hold (0: none)
     const float* screen_src = nullptr;
-    uint64_t split_gen = 0;     // data_gen whose fp16 pairs W_XSPLIT / W_XSINV hold (0: none)
+    uint64_t split_gen = 0;     // data_gen whose rows for the split W_XSPLIT / W_XSEXP hold (0: none)
     uint64_t split_order = 0;   // members_ver of their order (0: by row id)
-    bool split_bad = false;     // some |x|^2 of them is not finite
+    bool split_bad = false;     // some of them the inner product cannot take
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     void* scratch = nullptr;    // this device's fixed scratch array (gt_optimize_noalloc), or null
     std::string scratch_err;    // why it is null
@@ -304,8 +304,8 @@ enum Ws {
     W_OOC_A, W_OOC_B, W_OOC_C, W_OOC_D, W_OOC_E, W_OOC_F, W_OOC_G, W_CR, W_CRNORMS,
     W_KM_TRAIN, W_KM_MIND, W_KM_FLAG, W_KM_SEL, W_KM_POS, W_KM_SUMS, W_KM_NEW, W_KM_PSI, W_KM_P, W_KM_PN, W_KM_P8,
     W_KM_PN8, W_KM_OI, W_KM_OD, W_CH8, W_CHN, W_CHR, W_CHCNT, W_PAIRS, W_TOP2A, W_TOP2B, W_BUCKETD, W_KEY2,
-    W_BYKEY, W_BKTD, W_BOFF, W_SUBPOS, W_TOP2H, W_RV1, W_RV1M, W_XH, W_UBASE, W_UROWS, W_UITEMS, W_TQ, W_SQ, W_PAIRS2, W_XSPLIT, W_XSINV,
-    W_XSBAD, W_XSIOTA, W_XSPOS, W_COUNT_
+    W_BYKEY, W_BKTD, W_BOFF, W_SUBPOS, W_TOP2H, W_RV1, W_RV1M, W_XH, W_UBASE, W_UROWS, W_UITEMS, W_TQ, W_SQ, W_PAIRS2, W_XSPLIT, W_XSEXP,
+    W_XSBAD, W_XSPOS, W_QSPLIT, W_QSEXP, W_COUNT_
 };
 static_assert(W_COUNT_ <= 128, "workspace slots");
 
@@ -1117,27 +1117,28 @@ static void sub_order_members(Ctx& c, const DevMatrix& X, const Buckets& b, int 
     ++c.c->members_ver;
 }
 
-// The rows of X split into two fp16 parts (knn_wide_collect.hip) in the order
-// of the member list (null: their own), once per order; false where the copy
-// and the launch's candidate slots would not leave half of the free device
-// memory, or the inner product meets a row whose norm is not finite (the fp32
-// kernel then takes the launch).
+// The rows of X in the scale and order that the collect kernel for split rows
+// takes (knn_wide_collect.hip), by position in the member list (null: by row
+// id), once per order; false where the copy is beyond 64 GiB, or it and the
+// launch's candidate slots would not leave half of the free device memory, or
+// the inner product meets a row that it needs the fp32 kernel for.
 static bool split_rows(Ctx& c, const DevMatrix& X, const int32_t* d_members, int64_t rows, int metric)
 {
-    const int64_t N = X.N, Np = ceil_div(N, int64_t(32)) * 32;
-    const size_t need = static_cast<size_t>(Np) * X.Dp * 4, cand = static_cast<size_t>(rows + kQueriesPerWave) * kCollectCap * 8;
+    const int64_t N = X.N;
+    const size_t need = split_copy_bytes(N, X.Dp), cand = static_cast<size_t>(rows + kQueriesPerWave) * kCollectCap * 8;
     const size_t more = (c.c->ws[W_XSPLIT].cap < need ? need : 0) + (c.c->ws[W_CAND].cap < cand ? cand : 0);
+    if (need > size_t(16) << 32) return false;
     if (more > 0) {
         size_t fr = 0, total = 0;
         GT_HIP(hipMemGetInfo(&fr, &total));
         if (more > fr / 2) return false;
     }
-    uint16_t* xs = c.ws<uint16_t>(W_XSPLIT, need / 2);
-    float* inv = c.ws<float>(W_XSINV, static_cast<size_t>(N));
+    float* xs = c.ws<float>(W_XSPLIT, need / 4);
+    int32_t* ex = c.ws<int32_t>(W_XSEXP, static_cast<size_t>(N));
     unsigned int* bad = c.ws<unsigned int>(W_XSBAD, 1);
     const uint64_t order = d_members ? c.c->members_ver : 0;
     if (c.c->split_gen != c.c->data_gen || c.c->split_order != order) {
-        launch_split_rows(X.data, X.norms, d_members, N, X.Dp, xs, inv, bad, c.s);
+        launch_split_rows(X.data, X.norms, d_members, N, X.Dp, xs, ex, bad, c.s);
         c.c->split_gen = c.c->data_gen;
         c.c->split_order = order;
         c.c->split_bad = false;
@@ -1230,11 +1231,11 @@ static double bucketed_round(Ctx& c, const DevMatrix& X, const Buckets& b, int M
                              (scr == 2 || (scr == 1 && pairs_all >= static_cast<double>(int64_t(1) << 27)));
     const bool sub_ordered = own && !compact && c.c->dbg.sub_order != 0 && (!seed_d || want_prune || want_screen);
     if (sub_ordered) sub_order_members(c, X, b, metric, d_members);
-    // fp32 rows longer than 256: collect on the fp16 matrix cores over rows
-    // split in two, 256 or 128 queries per block (lists of 5..128 keys).
+    // fp32 rows longer than 256: collect on the bf16 matrix cores over rows
+    // split in three, 256 or 128 queries per block (lists of 5..128 keys).
     // (Rows of 161 to 256 stay on the fp32 kernel: its one chain of sums has
-    // errors of up to 4 ulps rms there, against 1 to 2.4 of the split rows,
-    // and 1.7 to 2.1 % of a table's positions, near ties, would change.)
+    // errors of up to 4 ulps rms there, and more exact sums would change 1.7
+    // to 2.1 % of a table's positions, near ties.)
     const bool wide = c.c->dbg.knn_collect != 0 && !use_i8(X, X, metric) && X.Dp > 256 && M > 4 && M <= 128 &&
                       split_rows(c, X, d_members, rows, metric);
     const int qstep = wide ? wide_queries_per_block(rows) : kQueriesPerBlock;
@@ -1244,10 +1245,8 @@ static double bucketed_round(Ctx& c, const DevMatrix& X, const Buckets& b, int M
     launch_copy_ranges(d_tasks, static_cast<int64_t>(tasks.size()), d_members, d_pool, c.s);
     int32_t* d_ppos = nullptr;   // wide: the pool entries' positions in the member list
     if (wide) {
-        int32_t* iota = c.ws<int32_t>(W_XSIOTA, static_cast<size_t>(N));
-        launch_iota(iota, N, c.s);
         d_ppos = c.ws<int32_t>(W_XSPOS, static_cast<size_t>(std::max<int64_t>(total, 1)));
-        launch_copy_ranges(d_tasks, static_cast<int64_t>(tasks.size()), iota, d_ppos, c.s);
+        launch_copy_ranges(d_tasks, static_cast<int64_t>(tasks.size()), nullptr, d_ppos, c.s);
     }
 
     std::vector<std::vector<WorkItem>> groups(static_cast<size_t>(C));
@@ -1427,7 +1426,9 @@ static double bucketed_round(Ctx& c, const DevMatrix& X, const Buckets& b, int M
                           screen_window, d_tq, d_urows, d_uitems, a.pairs_done, c.s);
         }
         if (wide) {
-            launch_wide_collect(a, qstep, c.ws<uint16_t>(W_XSPLIT, 0), c.ws<float>(W_XSINV, 0), d_ppos, false, c.s);
+            const float* xs = c.ws<float>(W_XSPLIT, 0);
+            const int32_t* ex = c.ws<int32_t>(W_XSEXP, 0);
+            launch_wide_collect(a, qstep, xs, ex, xs, ex, d_ppos, c.s);
             launch_collect_select(a, rows, c.s);
         } else if (collect) {
             launch_knn_collect_select(a, rows, c.s);
@@ -1481,61 +1482,83 @@ static double bucketed_round(Ctx& c, const DevMatrix& X, const Buckets& b, int M
     return t;
 }
 
-// Exact kNN of float rows on the fp16 matrix cores over rows split in two:
+// Exact kNN of float rows on the bf16 matrix cores over rows split in three:
 // the queries against the rows in slices of the pool (blocks of 256 queries,
-// two per CU in all), then each query's top k over its slices' candidates.
+// two per CU in all), then each query's top k over its slices' candidates;
+// kBatch queries at a time (as many as make 512 blocks by themselves), which
+// bounds the candidate slots to 256 MiB.
 // false: not this path's -- integer rows, short lists, few queries (the split
 // copy costs a pass over the rows, which below kMinQueries queries takes
 // longer than it saves), and rows of 129 to 256 dimensions, where the fp32
 // kernel's one chain of sums rounds most: it orders 1.1 to 1.6 % of a long
-// list's positions, near ties, otherwise than the split rows do (0.85 % at
+// list's positions, near ties, otherwise than more exact sums do (0.85 % at
 // 128, 0.2 % beyond 256), and callers keep the lists they have.
 static bool knn_exact_split(Ctx& c, const DevMatrix& X, const int32_t* d_q, int64_t nq, int k, int metric,
                             int32_t* out_ids, float* out_d)
 {
-    constexpr int64_t kMinQueries = 256, kMinRows = 4096, kSliceRows = 2048;
+    constexpr int64_t kMinQueries = 256, kMinRows = 4096, kSliceRows = 2048, kBatch = 512 * 256;
     if (c.c->dbg.knn_collect == 0 || use_i8(X, X, metric) || k <= 4 || k > 128 || nq < kMinQueries ||
         X.N < kMinRows || (X.Dp > 128 && X.Dp <= 256))
         return false;
     const int64_t by_pool = X.N / kSliceRows;
-    int64_t qpb = 256, qt = ceil_div(nq, qpb);
-    auto slices = [&]() { return std::max<int64_t>(1, std::min<int64_t>({512 / qt, by_pool, 128})); };
-    int64_t splits = slices();
-    if (qt * splits < 256) {
-        qpb = 128;
-        qt = ceil_div(nq, qpb);
-        splits = slices();
+    // slices of a batch of n queries in blocks of qpb
+    auto slices = [&](int64_t n, int64_t qpb) {
+        return std::max<int64_t>(1, std::min<int64_t>({512 / ceil_div(n, qpb), by_pool, kMaxSplits}));
+    };
+    auto block = [&](int64_t n) -> int64_t { return ceil_div(n, int64_t(256)) * slices(n, 256) < 256 ? 128 : 256; };
+    int64_t slots = 0;
+    for (int64_t b0 = 0; b0 < nq; b0 += kBatch) {
+        const int64_t n = std::min(kBatch, nq - b0);
+        slots = std::max(slots, slices(n, block(n)) * n);
     }
-    if (!split_rows(c, X, nullptr, splits * nq, metric)) return false;
-    const int64_t chunk = ceil_div(X.N, splits);
-    std::vector<WorkItem> items;
-    items.reserve(static_cast<size_t>(splits * qt + 8));
-    for (int64_t s = 0; s < splits; ++s)
-        for (int64_t t = 0; t < qt; ++t) {
-            WorkItem it{};
-            it.q_begin = t * qpb;
-            it.q_count = static_cast<int32_t>(std::min<int64_t>(qpb, nq - it.q_begin));
-            it.p_begin = s * chunk;
-            it.p_count = static_cast<int32_t>(std::max<int64_t>(0, std::min<int64_t>(chunk, X.N - it.p_begin)));
-            it.out_base = s * nq + it.q_begin;
-            items.push_back(it);
+    if (!split_rows(c, X, nullptr, slots, metric)) return false;
+    const float* xs = c.ws<float>(W_XSPLIT, 0);
+    const int32_t* ex = c.ws<int32_t>(W_XSEXP, 0);
+    uint64_t* cand = c.ws<uint64_t>(W_CAND, static_cast<size_t>(slots + kQueriesPerWave) * kCollectCap);
+    int32_t* cnt = c.ws<int32_t>(W_CANDCNT, static_cast<size_t>(slots));
+    for (int64_t b0 = 0; b0 < nq; b0 += kBatch) {
+        const int64_t n = std::min(kBatch, nq - b0), qpb = block(n), splits = slices(n, qpb), qt = ceil_div(n, qpb);
+        const int64_t chunk = ceil_div(X.N, splits);
+        // the batch's queries split in their own order (all rows: they are already)
+        const float* qs = xs;
+        const int32_t* qex = ex;
+        if (d_q) {
+            float* q = c.ws<float>(W_QSPLIT, split_copy_bytes(std::min(kBatch, nq), X.Dp) / 4);
+            int32_t* e = c.ws<int32_t>(W_QSEXP, static_cast<size_t>(std::min(kBatch, nq)));
+            launch_split_rows(X.data, X.norms, d_q + b0, n, X.Dp, q, e, c.ws<unsigned int>(W_XSBAD, 1), c.s);
+            qs = q;
+            qex = e;
         }
-    while (items.size() % 8 != 0) items.push_back(WorkItem{});   // q_count 0
-    WorkItem* d_items = c.ws<WorkItem>(W_ITEMS, items.size());
-    c.h2d(d_items, items.data(), items.size() * sizeof(WorkItem));
-    KnnArgs a{};
-    set_operands(a, X, X, metric);
-    a.q_rows = d_q;
-    a.items = d_items;
-    a.n_items = static_cast<int32_t>(items.size());
-    a.M = k;
-    a.metric = metric;
-    a.exclude_self = 1;
-    a.seed_ld = k;
-    a.cand = c.ws<uint64_t>(W_CAND, static_cast<size_t>(splits * nq + kQueriesPerWave) * kCollectCap);
-    a.cand_cnt = c.ws<int32_t>(W_CANDCNT, static_cast<size_t>(splits * nq));
-    launch_wide_collect(a, static_cast<int>(qpb), c.ws<uint16_t>(W_XSPLIT, 0), c.ws<float>(W_XSINV, 0), nullptr, true, c.s);
-    launch_split_select(a.cand, a.cand_cnt, nq, static_cast<int>(splits), k, out_ids, out_d, c.s);
+        const int64_t first = d_q ? 0 : b0;   // of the batch, in the query list
+        std::vector<WorkItem> items;
+        items.reserve(static_cast<size_t>(splits * qt + 8));
+        for (int64_t s = 0; s < splits; ++s)
+            for (int64_t t = 0; t < qt; ++t) {
+                WorkItem it{};
+                it.q_begin = first + t * qpb;
+                it.q_count = static_cast<int32_t>(std::min<int64_t>(qpb, n - t * qpb));
+                it.p_begin = s * chunk;
+                it.p_count = static_cast<int32_t>(std::max<int64_t>(0, std::min<int64_t>(chunk, X.N - it.p_begin)));
+                it.out_base = s * n + t * qpb;
+                items.push_back(it);
+            }
+        while (items.size() % 8 != 0) items.push_back(WorkItem{});   // q_count 0
+        WorkItem* d_items = c.ws<WorkItem>(W_ITEMS, items.size());
+        c.h2d(d_items, items.data(), items.size() * sizeof(WorkItem));
+        KnnArgs a{};
+        set_operands(a, X, X, metric);
+        a.q_rows = d_q ? d_q + b0 : nullptr;
+        a.items = d_items;
+        a.n_items = static_cast<int32_t>(items.size());
+        a.M = k;
+        a.metric = metric;
+        a.exclude_self = 1;
+        a.seed_ld = k;
+        a.cand = cand;
+        a.cand_cnt = cnt;
+        launch_wide_collect(a, static_cast<int>(qpb), xs, ex, qs, qex, nullptr, c.s);
+        launch_split_select(cand, cnt, n, static_cast<int>(splits), k, out_ids + b0 * k, out_d + b0 * k, c.s);
+    }
     return true;
 }
 

@@ -100,6 +100,7 @@ constexpr int kChunkRows = 64;       // pool rows per pruning chunk (= one colle
 constexpr int kMaxChunkWords = 24;   // pools of up to 24 * 32 chunks (49,152 rows) are pruned
 
 constexpr int kCollectCap = 256;   // candidate slots per query of a collect launch
+constexpr int kMaxSplits = 128;    // pool slices of an exact kNN launch
 
 // What a search launch reports over all of its queries.
 struct SearchTotals {

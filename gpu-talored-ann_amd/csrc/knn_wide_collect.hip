@@ -1,45 +1,54 @@
-// knn_wide_collect.hip -- collect + select kNN of fp32 rows on the fp16 matrix
-// cores over rows split in two: bucketed passes over rows longer than 256
+// knn_wide_collect.hip -- collect + select kNN of fp32 rows on the bf16 matrix
+// cores over rows split in three: bucketed passes over rows longer than 256
 // floats, and exact kNN of many queries over rows of up to 128 or more than
 // 256
 // (src/bucket.cu:4101-4265 top-M semantics: self excluded, (-1, +inf)
 // padding, ties by id).
 //
 // The split.  Row x is scaled by a power of two of its own, 2^k with
-// max |x_i| 2^k in [2^14, 2^15), and every element written as h + m: h the
-// fp16 nearest to it, m the fp16 nearest to the rest.  h keeps 11 bits and a
-// sign, m the next 11, so h + m is the fp32 element to within half of its
-// last bit (2^-24 of the element; where m is subnormal, flushed or not,
-// within 2^-29 of the row's largest).  A dot product is the sum of h h, h m and m h
-// products, each exact in the fp32 accumulator (v_mfma_f32_32x32x16_f16);
-// the m m products left out are at most 2^-24 of their terms.  Both are
-// below the roundings of an fp32 sum over D terms: measured against 64 bits on
-// D 288..1024 (tests/test_gpu_wide_split.py) the distances are as close as
-// those of the fp32 kernel (knn_wide_kernel; 1.59 and 1.60 ulps rms at D 960),
-// and closer than knn_fused_kernel's (1.9 and 3.1 at D 128).  Integer-valued rows below 2^11
-// have m = 0 and give exact sums.
+// |x| 2^k in [2^56, 2^57), and every element written as h + m + l: h the bf16
+// nearest to it, m the bf16 nearest to the rest, l what is left.  Each takes
+// the next 8 of the element's 24 bits, so the three are the element exactly
+// (while it is above 2^-110 of |x|: l is then a normal number).  A dot product
+// is the sum of the products h h, h m, m h, h l, l h and m m, each exact in
+// the fp32 accumulator (v_mfma_f32_32x32x16_bf16); the three left out are at
+// most 2^-26 of their terms, a quarter of a product's own rounding in fp32.
+// So nothing is lost whatever the rows hold: few dimensions, few non-zeros,
+// whole numbers (products below 2^24 have no part in those left out: one
+// factor is below 2^12 and then has no l, and has no m where the other has an
+// l).  Two fp16 parts and three products, half the matrix work, lose the
+// element's last bit and m m: a row of one element 3001 then lay at distance 2
+// from its own duplicate, and rows of 1 to 4 elements had twice the fp32
+// kernel's error.  Measured against 64 bits (tests/test_gpu_wide_split.py,
+// tests/test_gpu_knn_exact_split.py): never above the fp32 kernels' error.
+// The inner product asks for every term's own bits: there a row with a
+// non-zero element below 2^-105 of |x| (a product of two could leave a part
+// below the normal numbers), or a norm that is not finite, sends the launch to
+// the fp32 kernel.  L2 keys add |q|^2 + |p|^2, whose rounding is far above.
 // A row with an element that is not finite has a norm that is not finite
 // either: its L2 keys are +inf or NaN, which no list takes, whatever its dot
-// products (the inner product of such rows stays on the fp32 kernel).
+// products.
 //
-// Three fp16 products cost 3/16 of one fp32 product of the fp32 matrix cores,
-// and h and m take the fp32 row's bytes, so moving rows is what there is to
-// save: a block is 8 waves with 256 queries (32 per wave, read from L2 chunk
-// by chunk) against 192 or 256 pool rows at a time (32-dimension chunks
-// double-buffered in LDS, shared by the waves; 6 or 8 accumulator tiles of
-// 32 x 32 per wave).  Launches with fewer blocks than the chip has CUs take 4
-// waves and 128 queries.  What bounds it (D 960, 2.1e9 pairs, keys not
-// collected, variants timed with parts left out): 13.3 ms, without the query
-// loads 11.2, without the pool loads 12.1, without either and the barrier 9.2,
-// the MFMAs alone 4.9: the LDS reads (every wave reads every pool row), then
-// the loads' latency.  Stages of two chunks, half the barriers, were no faster.
-// Measured (bucketed pass over 100,003 x 960, 25 buckets, one probe, M 96):
-// 20.3 ms on the fp32 kernel, 8.3 here; a 10^6 x 960 build 237 -> 128 ms; exact
-// 100-NN of 10,000 queries in 1,000,003 x 100: 40.2 -> 14.1 ms.
-//
+// Six bf16 products cost 6/16 of one fp32 product of the fp32 matrix cores.
+// Rows move as scaled floats, in an order of their own (piece_at), and are
+// split on their way into LDS and into the query operands while the matrix
+// cores are busy: a block is 8 waves with 256 queries (32 per wave, read from
+// L2 chunk by chunk) against 192 pool rows at a time (32-dimension chunks
+// double-buffered in LDS, shared by the waves; 6 accumulator tiles of 32 x 32
+// per wave).  Launches with fewer blocks than the chip has CUs take 4 waves
+// and 128 queries.  A copy of the three parts, 6 bytes per element, was
+// slower: bucketed pass below 13.0 ms, build 187.
+// What bounds it (bucketed pass over 100,003 x 960, 25 buckets, one probe, M
+// 96; counters): where a CU has a block, its matrix cores are busy 57 % of the
+// time; they wait for the sums' 32 additions per tile, the split and the
+// barrier of each chunk.  Over the launch 30 %: some 400 blocks, a bucket's on
+// one XCD, hold the 256 CUs 52 % of the time.
+// Measured: that pass 20.3 ms on the fp32 kernel, 12.4 here; a 10^6 x 960
+// build 241 -> 172 ms; exact 100-NN of 10,000 queries in 1,000,003 x 100:
+// 40.3 -> 20.1 ms.  (With two fp16 parts, which lose bits: 8.4, 128 and 13.8.)
 // Keys at or below a query's threshold go to its candidate slots in HBM as in
 // knn_collect.hip.  An unseeded pass first bounds each query's M-th smallest
-// key by bisection over the 256 keys of the first pool tile, which the lane
+// key by bisection over the 192 keys of the first pool tile, which the lane
 // pair holds in registers.
 #include "collect_device.hpp"
 
@@ -47,137 +56,127 @@
 
 namespace gtann {
 
-typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
-constexpr int kMaxSplits = 128;   // pool slices of an exact kNN launch
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));   // a value: never memory
 
-typedef _Float16 halfx4 __attribute__((ext_vector_type(4)));
+constexpr int kSplitChunk = 32;   // dimensions per chunk
+constexpr int kSplitRows = 192;   // pool rows per tile: six accumulators per wave
+constexpr int kSplitTiles = kSplitRows / kPoolTile;
+constexpr int kRowPieces = kSplitChunk / 4;            // 16-byte pieces of a row's chunk in the copy: 4 floats
+constexpr int kTilePieces = 3 * kSplitChunk / 8;       // and in LDS: 8 h of each quarter, then m, then l
 
-constexpr int kSplitChunk = 32;                   // dimensions per chunk: 32 h, then 32 m
-
-// Pool rows per tile.  Rows of up to 256 dimensions sum all chunks in one
-// accumulator (their error is below the fp32 kernel's as it is); longer ones
-// sum each chunk on its own, which takes the registers of a quarter of the
-// tile (D 960, error against 64 bits: 4.8 ulps rms in one accumulator, 1.6 by
-// chunks, 1.6 the fp32 kernel).
-template <bool PARTS>
-struct SplitTile {
-    static constexpr int ROWS = PARTS ? 192 : 256;
-    static constexpr int TILES = ROWS / kPoolTile;
-};
-constexpr int kSplitStride = 2 * kSplitChunk + 8; // halves per LDS row: 16 rows' same pieces fill the banks once
-
-// Where the split copy holds chunk c of the row at position p of the member
-// list: groups of 32 positions, chunk-major, so that a tile's chunk is a few
-// whole 4 KiB pieces (by row id, a 128-byte piece of a row in 512 places per
-// chunk, the launch took 2.1 times as long).
-__device__ __forceinline__ int64_t split_at(int64_t p, int c, int nch)
+// Where the copy of the rows holds piece 0 of chunk 0 of the row at position
+// p, in pieces: groups of 32 positions, chunk-major, a chunk's pieces one
+// after another, each for the group's 32 rows.  A tile's chunk is then a few
+// whole 4 KiB blocks, and 32 lanes with consecutive rows read 512 consecutive
+// bytes.
+__device__ __forceinline__ uint32_t piece_at(uint32_t p, int nch)
 {
-    return (((p >> 5) * nch + c) * 32 + (p & 31)) * 2 * kSplitChunk;
+    return (p >> 5) * static_cast<uint32_t>(nch * kRowPieces * 32) + (p & 31u);
 }
 
-// The rows X[members[p]] (stride Dp; members null: X[p]) to Xs at their positions p: per row and
-// chunk 32 h, then 32 m; inv[p] = 2^-k.  *bad counts rows whose |x|^2 is not
-// finite.  One wave per position.
+// The rows X[members[p]] (stride Dp; members null: X[p]), scaled, to Xs at
+// their positions p; ex[p] = -k.  *bad is set by rows that the inner product
+// cannot take.  One block per 32 positions, eight lanes per row.
 __global__ void __launch_bounds__(256) split_rows_kernel(const float* __restrict__ X, const float* __restrict__ nrm,
                                                          const int32_t* __restrict__ members, int64_t N, int Dp,
-                                                         _Float16* __restrict__ Xs, float* __restrict__ inv,
+                                                         f32x4* __restrict__ Xs, int32_t* __restrict__ ex,
                                                          unsigned int* __restrict__ bad)
 {
-    const int lane = threadIdx.x & 63;
-    const int64_t pos = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
+    const int piece = threadIdx.x & 7;
+    const int64_t pos = static_cast<int64_t>(blockIdx.x) * 32 + (threadIdx.x >> 3);
     if (pos >= N) return;
     const int64_t row = members ? members[pos] : pos;
-    const float4* x = reinterpret_cast<const float4*>(X + row * Dp);
-    const int n4 = Dp >> 2;
-    float4 v[4];                                   // Dp <= 1024: four float4 per lane
-    float mx = 0.f;
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-        v[t] = lane + 64 * t < n4 ? x[lane + 64 * t] : make_float4(0.f, 0.f, 0.f, 0.f);
-        mx = fmaxf(fmaxf(fmaxf(mx, fabsf(v[t].x)), fmaxf(fabsf(v[t].y), fabsf(v[t].z))), fabsf(v[t].w));
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
-    int e = 0;
-    const bool finite = mx < INFINITY;
-    if (finite && mx > 0.f) frexpf(mx, &e);        // mx < 2^e
-    // (at most 2^126: the scale back stays a normal float; every float element
-    // is then a multiple of 2^-23, which the two parts hold as well)
-    const int k = finite && mx > 0.f ? min(15 - e, 126) : 0;
-    auto scaled = [&](float y) -> float { return finite ? ldexpf(y, k) : 0.f; };
+    const f32x4* x = reinterpret_cast<const f32x4*>(X + row * Dp) + piece;
+    const float n = nrm[row];
+    const bool finite = n < INFINITY;
+    // |x| < 2^e; norms too small to be exact: every element is below 2^-50
+    int e = -50;
+    if (finite && n >= 0x1p-100f) frexpf(sqrtf(n), &e);
+    const int k = finite ? 57 - e : 0;
     const int nch = Dp / kSplitChunk;
+    f32x4* out = Xs + piece_at(static_cast<uint32_t>(pos), nch) + piece * 32;
+    bool tiny = !finite;
+    constexpr int U = 4;
+    for (int c0 = 0; c0 < nch; c0 += U) {
+        f32x4 v[U];
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-        const int q = lane + 64 * t;
-        if (q < n4) {
-            const float y[4] = {scaled(v[t].x), scaled(v[t].y), scaled(v[t].z), scaled(v[t].w)};
-            halfx4 h, m;
+        for (int u = 0; u < U; ++u) v[u] = x[kRowPieces * min(c0 + u, nch - 1)];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (c0 + u >= nch) break;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                h[i] = static_cast<_Float16>(y[i]);
-                m[i] = static_cast<_Float16>(y[i] - static_cast<float>(h[i]));
+                v[u][i] = finite ? ldexpf(v[u][i], k) : 0.f;
+                tiny = tiny || (v[u][i] != 0.f && fabsf(v[u][i]) < 0x1p-48f);
             }
-            const int d = 4 * q;                   // dims d .. d + 3 of chunk d / 32
-            _Float16* c = Xs + split_at(pos, d / kSplitChunk, nch) + d % kSplitChunk;
-            *reinterpret_cast<halfx4*>(c) = h;
-            *reinterpret_cast<halfx4*>(c + kSplitChunk) = m;
+            out[(c0 + u) * kRowPieces * 32] = v[u];
         }
     }
-    if (lane == 0) {
-        inv[pos] = ldexpf(1.f, -k);
-        if (!(nrm[row] < INFINITY)) atomicAdd(bad, 1u);
-    }
+    if (piece == 0) ex[pos] = -k;
+    if (__ballot(tiny) && (threadIdx.x & 63) == 0) atomicOr(bad, 1u);
 }
 
 __global__ void split_clear_kernel(unsigned int* bad) { *bad = 0u; }
 
-void launch_split_rows(const float* X, const float* nrm, const int32_t* members, int64_t N, int Dp, uint16_t* Xs,
-                       float* inv, unsigned int* bad, hipStream_t s)
+// Bytes of the copy of n rows
+size_t split_copy_bytes(int64_t n, int Dp)
 {
-    GT_REQUIRE(Dp % kSplitChunk == 0 && Dp <= 1024, "split rows: padded dimension");
+    return static_cast<size_t>(ceil_div(n, int64_t(32)) * 32) * Dp * sizeof(float);
+}
+
+void launch_split_rows(const float* X, const float* nrm, const int32_t* members, int64_t N, int Dp, float* Xs,
+                       int32_t* ex, unsigned int* bad, hipStream_t s)
+{
+    GT_REQUIRE(Dp % kSplitChunk == 0 && Dp <= 1024 && split_copy_bytes(N, Dp) <= size_t(16) << 32, "split rows: sizes");
     hipLaunchKernelGGL(split_clear_kernel, dim3(1), dim3(1), 0, s, bad);
     if (N > 0)
-        hipLaunchKernelGGL(split_rows_kernel, dim3(static_cast<unsigned>(ceil_div(N, int64_t(4)))), dim3(256), 0, s, X,
-                           nrm, members, N, Dp, reinterpret_cast<_Float16*>(Xs), inv, bad);
+        hipLaunchKernelGGL(split_rows_kernel, dim3(static_cast<unsigned>(ceil_div(N, int64_t(32)))), dim3(256), 0, s, X,
+                           nrm, members, N, Dp, reinterpret_cast<f32x4*>(Xs), ex, bad);
     GT_HIP(hipGetLastError());
 }
 
-__global__ void __launch_bounds__(256) iota_kernel(int32_t* p, int64_t n)
+// Floats as sums of three bf16: h the nearest to it, m the nearest to the
+// rest, l what is left; elements 2 i and 2 i + 1 in word i of each part.
+__device__ __forceinline__ void split4(const f32x4& z, u32x2 (&part)[3])
 {
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-    if (i < n) p[i] = static_cast<int32_t>(i);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        f32x2 r = {z[2 * i], z[2 * i + 1]};
+#pragma unroll
+        for (int x = 0; x < 3; ++x) {
+            const uint32_t p = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, bf16x2));
+            part[x][i] = p;
+            r = f32x2{r[0] - __uint_as_float(p << 16), r[1] - __uint_as_float(p & 0xFFFF0000u)};
+        }
+    }
 }
 
-void launch_iota(int32_t* p, int64_t n, hipStream_t s)
-{
-    if (n <= 0) return;
-    hipLaunchKernelGGL(iota_kernel, dim3(static_cast<unsigned>(ceil_div(n, int64_t(256)))), dim3(256), 0, s, p, n);
-    GT_HIP(hipGetLastError());
-}
-
-template <int NW, bool PARTS>
+template <int NW>
 struct WideCollectSmem {
-    static constexpr int kSplitRows = SplitTile<PARTS>::ROWS;
-    _Float16 tile[2][kSplitRows][kSplitStride];
+    __bf16 tile[2][kSplitTiles * kTilePieces * 32 * 8];   // 32-row blocks: a piece's 32 rows one after another
     float tnorm[2][kSplitRows];     // |p|^2 (L2) or 0 (IP); +inf past the slice end
-    float tinv[2][kSplitRows];      // 2^-k of the row
+    int32_t tex[2][kSplitRows];     // -k of the row
     int32_t trow[2][kSplitRows];    // pool row id, -1 past the slice end
     CollectWave wv[NW];
 };
 
-template <int METRIC, int NW, bool PARTS>
+template <int METRIC, int NW>
 __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW == 8 ? 2 : 1)))
-knn_wide_collect_kernel(KnnArgs a, const _Float16* __restrict__ Xs, const float* __restrict__ inv,
-                        const int32_t* __restrict__ p_pos, int q_by_row)
+knn_wide_collect_kernel(KnnArgs a, const f32x4* __restrict__ Xs, const int32_t* __restrict__ ex,
+                        const f32x4* __restrict__ Qs, const int32_t* __restrict__ qex,
+                        const int32_t* __restrict__ p_pos)
 {
     extern __shared__ __align__(16) unsigned char smem[];
-    using Smem = WideCollectSmem<NW, PARTS>;
+    using Smem = WideCollectSmem<NW>;
     Smem& sm = *reinterpret_cast<Smem*>(smem);
-    constexpr int kSplitRows = SplitTile<PARTS>::ROWS, kSplitTiles = SplitTile<PARTS>::TILES;
     constexpr int T = 64 * NW;
-    constexpr int PT = kSplitRows * 8 / T;          // 16-byte pieces of a chunk's rows per thread
-    static_assert(PT * T == kSplitRows * 8, "whole pieces");
-    constexpr int RS = T / 8;                       // rows between a thread's pieces
+    constexpr int PT = kSplitRows * kRowPieces / T;   // pieces of a chunk's rows per thread
+    static_assert(PT * T == kSplitRows * kRowPieces && T % 256 == 0 && PT % 3 == 0, "a thread's pieces are of one row and place");
 
     const int per = a.n_items / 8;
     const int item_idx = static_cast<int>(blockIdx.x % 8) * per + static_cast<int>(blockIdx.x / 8);
@@ -194,8 +193,8 @@ knn_wide_collect_kernel(KnnArgs a, const _Float16* __restrict__ Xs, const float*
     const int64_t qi = it.q_begin + qlocal;
     const int32_t qrow = qvalid ? (a.q_rows ? a.q_rows[qi] : static_cast<int32_t>(qi)) : 0;
     const float qn = (qvalid && METRIC == 0) ? a.nq[qrow] : 0.f;
-    const int64_t qpos = q_by_row ? qrow : qvalid ? qi : it.q_begin;
-    const float qinv = inv[qpos];
+    const int64_t qpos = qvalid ? qi : it.q_begin;
+    const int qe = qex[qpos];
 
     CollectState st;
     float seed = FLT_MAX;
@@ -212,72 +211,84 @@ knn_wide_collect_kernel(KnnArgs a, const _Float16* __restrict__ Xs, const float*
 
     const int pcount = it.p_count;
     const int nst = (pcount + kSplitRows - 1) / kSplitRows;
-    // the pool-list entry scanned at p (< pcount)
-    auto pool_at = [&](int p) -> int64_t {
-        p += it.p_rot;
-        if (p >= pcount) p -= pcount;
-        return it.p_begin + p;
-    };
 
-    // thread tid stages 16-byte piece tid % 8 of rows tid / 8 + RS u (rows past
-    // the slice hold the last row's values: their norm is +inf and their id -1)
-    const int piece = tid & 7, r0 = tid >> 3;
-    int32_t rid[PT], rid_n[PT];   // their positions in the member list
-    uint4 pre[PT];
-    auto set_ids = [&](int stile, int32_t (&ids)[PT]) {
+    // thread tid stages piece tid / 32 % 8 of row tid % 32 of the 32-row blocks
+    // tid / 256 + T / 256 u (rows past the slice hold the last row's values:
+    // their norm is +inf and their id -1)
+    const int piece = (tid >> 5) & 7;
+    uint32_t at[PT], at_n[PT];   // of this tile and the next: the pieces of chunk 0
+    f32x4 pre[PT];
+    auto set_at = [&](int stile, uint32_t (&o)[PT]) {
 #pragma unroll
         for (int u = 0; u < PT; ++u) {
-            const int64_t pl = pool_at(min(stile * kSplitRows + r0 + RS * u, pcount - 1));
-            ids[u] = p_pos ? p_pos[pl] : static_cast<int32_t>(pl);
+            const int r = 32 * (tid / 256 + T / 256 * u) + j;
+            const int64_t pl = it.p_begin + min(stile * kSplitRows + r, pcount - 1);
+            o[u] = piece_at(static_cast<uint32_t>(p_pos ? p_pos[pl] : pl), nch) + 32 * piece;
         }
     };
     auto load_pool = [&](bool next, int c) {
 #pragma unroll
-        for (int u = 0; u < PT; ++u) {
-            const int32_t p = next ? rid_n[u] : rid[u];
-            const uint4 v = *reinterpret_cast<const uint4*>(Xs + split_at(p, c, nch) + 8 * piece);
-            pre[u] = make_uint4(v.x, v.y, v.z, v.w);
+        for (int u = 0; u < PT; ++u) pre[u] = Xs[(next ? at_n[u] : at[u]) + static_cast<uint32_t>(c * kRowPieces * 32)];
+    };
+    auto store_pool = [&](int buf, int u) {
+        u32x2 part[3];
+        asm volatile("" : "+v"(pre[u]));   // not before here
+        split4(pre[u], part);
+        u32x2* t = reinterpret_cast<u32x2*>(sm.tile[buf]) + (tid / 256 + T / 256 * u) * (kTilePieces * 64) +
+                    (piece >> 1) * 64 + 2 * j + (piece & 1);
+#pragma unroll
+        for (int x = 0; x < 3; ++x) t[x * 4 * 64] = part[x];
+    };
+    // the query's chunk: h of dims 8 h.., 16 + 8 h.., then m, then l
+    const f32x4* qrow0 = Qs + piece_at(static_cast<uint32_t>(qpos), nch) + 64 * h;
+    bf16x8 qc[6];
+    f32x4 qx[4];
+    auto load_q = [&](int c) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) qx[s] = qrow0[static_cast<uint32_t>(c * kRowPieces * 32 + (s >> 1) * 128 + (s & 1) * 32)];
+    };
+    auto split_q = [&]() {
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            u32x2 a0[3], a1[3];
+            asm volatile("" : "+v"(qx[2 * s]), "+v"(qx[2 * s + 1]));   // not before here
+            split4(qx[2 * s], a0);
+            split4(qx[2 * s + 1], a1);
+#pragma unroll
+            for (int x = 0; x < 3; ++x) qc[2 * x + s] = __builtin_bit_cast(bf16x8, u32x4{a0[x][0], a0[x][1], a1[x][0], a1[x][1]});
         }
     };
-    auto store_pool = [&](int buf) {
-#pragma unroll
-        for (int u = 0; u < PT; ++u) *reinterpret_cast<uint4*>(&sm.tile[buf][r0 + RS * u][8 * piece]) = pre[u];
-    };
-    // the query's chunk: h of dims 8h.., 16 + 8h.., then m
-    halfx8 qc[4], qx[4];
-    auto load_q = [&](int c, halfx8 (&dst)[4]) {
-#pragma unroll
-        for (int s = 0; s < 4; ++s) dst[s] = *reinterpret_cast<const halfx8*>(Xs + split_at(qpos, c, nch) + 8 * h + 16 * s);
-    };
-    // ids, norms and scales of tile stile's row tid
-    auto tile_meta = [&](int stile, int32_t& id, float& n, float& iv) {
+    // id, norm and scale of tile stile's row tid
+    auto tile_meta = [&](int stile, int32_t& id, float& n, int32_t& x) {
         id = -1;
         n = INFINITY;
-        iv = 1.f;
+        x = 0;
         const int p = stile * kSplitRows + tid;
         if (tid < kSplitRows && p < pcount) {
-            const int64_t pl = pool_at(p);
+            const int64_t pl = it.p_begin + p;
             id = a.p_rows ? a.p_rows[pl] : static_cast<int32_t>(pl);
             n = METRIC == 0 ? a.np[id] : 0.f;
-            iv = inv[p_pos ? p_pos[pl] : pl];
+            x = ex[p_pos ? p_pos[pl] : pl];
         }
     };
-    static_assert(T >= kSplitRows || T == 256, "one row's ids per thread");
+    static_assert(T >= kSplitRows, "one row's ids per thread");
 
     if (nst > 0) {
-        set_ids(0, rid);
-        set_ids(1, rid_n);
-        int32_t nrow;
-        float nnrm, ninv;
-        tile_meta(0, nrow, nnrm, ninv);
+        set_at(0, at);
+        set_at(1, at_n);
+        int32_t nrow, nex;
+        float nnrm;
+        tile_meta(0, nrow, nnrm, nex);
         if (tid < kSplitRows) {
             sm.trow[0][tid] = nrow;
             sm.tnorm[0][tid] = nnrm;
-            sm.tinv[0][tid] = ninv;
+            sm.tex[0][tid] = nex;
         }
         load_pool(false, 0);
-        store_pool(0);
-        load_q(0, qc);
+        load_q(0);
+#pragma unroll
+        for (int u = 0; u < PT; ++u) store_pool(0, u);
+        split_q();
         __syncthreads();
     }
 
@@ -288,52 +299,67 @@ knn_wide_collect_kernel(KnnArgs a, const _Float16* __restrict__ Xs, const float*
         for (int u = 0; u < kSplitTiles; ++u)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[u][r] = 0.f;
-        int32_t nrow;
-        float nnrm, ninv;
-        tile_meta(stile + 1, nrow, nnrm, ninv);
+        int32_t nrow, nex;
+        float nnrm;
+        tile_meta(stile + 1, nrow, nnrm, nex);
 #pragma unroll 1
         for (int c = 0; c < nch; ++c) {
             const int buf = g & 1;
             const bool last = c + 1 == nch;
             load_pool(last, last ? 0 : c + 1);
-            load_q(last ? 0 : c + 1, qx);
+            load_q(last ? 0 : c + 1);
             // the next chunk's loads stay ahead of this chunk's MFMAs
             __builtin_amdgcn_sched_barrier(0);
-            // A = pool row u*32 + (lane%32), B = query lane%32, the small
-            // products first; PARTS: the chunk's sum is added to the running
-            // dot, so that the rounding error grows with sqrt(chunks)
+            // A = pool row u*32 + (lane%32), B = query lane%32.  The h h sums
+            // and the smaller products are kept apart and added in fp32
+            // instructions, which round to nearest: the matrix cores cut what
+            // they add off below the largest term (single products of rows of
+            // one element: 0.42 ulps rms with one sum, 0.29 in fp32).  The
+            // chunk's sum is added to the running dot, so that the rounding
+            // error grows with sqrt(chunks)
 #pragma unroll
             for (int u = 0; u < kSplitTiles; ++u) {
-                halfx8 av[4];
+                bf16x8 av[6];
 #pragma unroll
-                for (int s = 0; s < 4; ++s)
-                    av[s] = *reinterpret_cast<const halfx8*>(&sm.tile[buf][kPoolTile * u + j][8 * h + 16 * s]);
-                floatx16 part;
+                for (int s = 0; s < 6; ++s)
+                    av[s] = *reinterpret_cast<const bf16x8*>(&sm.tile[buf][8 * (32 * (kTilePieces * u + 2 * s + h) + j)]);
+                floatx16 part, top;
 #pragma unroll
-                for (int r = 0; r < 16; ++r) part[r] = PARTS ? 0.f : acc[u][r];
-                part = __builtin_amdgcn_mfma_f32_32x32x16_f16(av[2], qc[0], part, 0, 0, 0);
-                part = __builtin_amdgcn_mfma_f32_32x32x16_f16(av[3], qc[1], part, 0, 0, 0);
-                part = __builtin_amdgcn_mfma_f32_32x32x16_f16(av[0], qc[2], part, 0, 0, 0);
-                part = __builtin_amdgcn_mfma_f32_32x32x16_f16(av[1], qc[3], part, 0, 0, 0);
-                part = __builtin_amdgcn_mfma_f32_32x32x16_f16(av[0], qc[0], part, 0, 0, 0);
-                part = __builtin_amdgcn_mfma_f32_32x32x16_f16(av[1], qc[1], part, 0, 0, 0);
+                for (int r = 0; r < 16; ++r) part[r] = top[r] = 0.f;
+                auto product = [&](floatx16& sum, int x, int y) __attribute__((always_inline)) {
+                    sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[2 * x], qc[2 * y], sum, 0, 0, 0);
+                    sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[2 * x + 1], qc[2 * y + 1], sum, 0, 0, 0);
+                };
+                product(part, 2, 0);
+                product(part, 0, 2);
+                product(part, 1, 1);
+                product(part, 1, 0);
+                product(part, 0, 1);
+                product(top, 0, 0);
+                // the next chunk is split while the matrix cores are busy
+                if (u >= 2 && u < 5) {
 #pragma unroll
-                for (int r = 0; r < 16; ++r) acc[u][r] = PARTS ? acc[u][r] + part[r] : part[r];
+                    for (int i = 0; i < PT / 3; ++i) store_pool(buf ^ 1, PT / 3 * (u - 2) + i);
+                }
+                if (u == 5) split_q();
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[u][r] += top[r] + part[r];
+                // the sums of one tile at a time: the compiler would put all
+                // six off to the end, in registers that there are not
+                asm volatile("" : "+v"(acc[u]));
+                __builtin_amdgcn_sched_barrier(0x104);
             }
-            store_pool(buf ^ 1);
             __syncthreads();
-#pragma unroll
-            for (int s = 0; s < 4; ++s) qc[s] = qx[s];
             ++g;
         }
         if (tid < kSplitRows) {
             sm.trow[(stile + 1) & 1][tid] = nrow;
             sm.tnorm[(stile + 1) & 1][tid] = nnrm;
-            sm.tinv[(stile + 1) & 1][tid] = ninv;
+            sm.tex[(stile + 1) & 1][tid] = nex;
         }
 #pragma unroll
-        for (int u = 0; u < PT; ++u) rid[u] = rid_n[u];
-        set_ids(stile + 2, rid_n);
+        for (int u = 0; u < PT; ++u) at[u] = at_n[u];
+        set_at(stile + 2, at_n);
 
         // the keys, in place: lane (j, h) holds rows 8g + 4h + e of every tile
         const int sb = stile & 1;
@@ -342,18 +368,18 @@ knn_wide_collect_kernel(KnnArgs a, const _Float16* __restrict__ Xs, const float*
 #pragma unroll
             for (int gg = 0; gg < 4; ++gg) {
                 const float4 pn = *reinterpret_cast<const float4*>(&sm.tnorm[sb][kPoolTile * u + 8 * gg + 4 * h]);
-                const float4 pi = *reinterpret_cast<const float4*>(&sm.tinv[sb][kPoolTile * u + 8 * gg + 4 * h]);
-                const float n4[4] = {pn.x, pn.y, pn.z, pn.w}, i4[4] = {pi.x, pi.y, pi.z, pi.w};
+                const int4 pe = *reinterpret_cast<const int4*>(&sm.tex[sb][kPoolTile * u + 8 * gg + 4 * h]);
+                const float n4[4] = {pn.x, pn.y, pn.z, pn.w};
+                const int e4[4] = {pe.x, pe.y, pe.z, pe.w};
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    // powers of two: exact (their product alone may underflow where the dot does not)
-                    const float dot = (acc[u][4 * gg + e] * qinv) * i4[e];
+                    const float dot = ldexpf(acc[u][4 * gg + e], qe + e4[e]);
                     acc[u][4 * gg + e] = METRIC == 0 ? fmaf(-2.f, dot, n4[e] + qn) : fmaf(-1.f, dot, n4[e]);
                 }
             }
         if (stile == 0 && !a.seed_d) {
             // a bound on the M-th smallest key: bisection between the
-            // smallest and the largest of the pair's 256 keys (the query
+            // smallest and the largest of the pair's 192 keys (the query
             // itself among them: one more than M keys at or below it)
             float lo = INFINITY, hi = -INFINITY;
             int n = 0;
@@ -591,34 +617,28 @@ void launch_split_select(const uint64_t* cand, const int32_t* cnt, int64_t nq, i
 // that gives every CU a block, else 128.
 int wide_queries_per_block(int64_t n_queries) { return n_queries >= int64_t(256) * 256 ? 256 : 128; }
 
-// Xs, inv: the split rows by position; p_pos: the position of every pool-list
-// entry (null: itself).  Query i's position is i, its place in the member list
-// a.q_rows, or with q_by_row its row id (rows split in their own order).
-void launch_wide_collect(const KnnArgs& a, int qpb, const uint16_t* Xs, const float* inv, const int32_t* p_pos,
-                         bool q_by_row, hipStream_t s)
+// Xs, ex: the split rows by position; p_pos: the position of every pool-list
+// entry (null: itself).  Qs, qex: the split queries, query i (its place in
+// a.q_rows) at position i.
+void launch_wide_collect(const KnnArgs& a, int qpb, const float* Xs, const int32_t* ex, const float* Qs,
+                         const int32_t* qex, const int32_t* p_pos, hipStream_t s)
 {
     GT_REQUIRE((p_pos != nullptr) == (a.p_rows != nullptr) && a.n_items % 8 == 0 && a.Dp % kSplitChunk == 0 && a.cand && a.cand_cnt && (qpb == 128 || qpb == 256),
                "wide collect launch");
     if (a.n_items <= 0) return;
-    const _Float16* x = reinterpret_cast<const _Float16*>(Xs);
     auto go = [&](auto kernel, int waves, size_t lds) {
         GT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                    static_cast<int>(lds)));
         hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(a.n_items)), dim3(static_cast<unsigned>(64 * waves)), lds, s,
-                           a, x, inv, p_pos, q_by_row ? 1 : 0);
+                           a, reinterpret_cast<const f32x4*>(Xs), ex, reinterpret_cast<const f32x4*>(Qs), qex, p_pos);
     };
-    auto by_metric = [&](auto nw, auto parts) {
+    auto by_metric = [&](auto nw) {
         constexpr int NW = decltype(nw)::value;
-        constexpr bool P = decltype(parts)::value;
-        if (a.metric == 0) go(&knn_wide_collect_kernel<0, NW, P>, NW, sizeof(WideCollectSmem<NW, P>));
-        else go(&knn_wide_collect_kernel<1, NW, P>, NW, sizeof(WideCollectSmem<NW, P>));
+        if (a.metric == 0) go(&knn_wide_collect_kernel<0, NW>, NW, sizeof(WideCollectSmem<NW>));
+        else go(&knn_wide_collect_kernel<1, NW>, NW, sizeof(WideCollectSmem<NW>));
     };
-    auto by_dim = [&](auto nw) {
-        if (a.Dp > 256) by_metric(nw, std::true_type{});
-        else by_metric(nw, std::false_type{});
-    };
-    if (qpb == 256) by_dim(std::integral_constant<int, 8>{});
-    else by_dim(std::integral_constant<int, 4>{});
+    if (qpb == 256) by_metric(std::integral_constant<int, 8>{});
+    else by_metric(std::integral_constant<int, 4>{});
     GT_HIP(hipGetLastError());
 }
 

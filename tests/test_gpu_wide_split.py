@@ -1,8 +1,8 @@
 """Bucketed kNN of float rows longer than 256: the collect kernel on rows
-split into two fp16 parts (shorter rows: the fp32 kernels on both sides), against the merging fp32 kernels (knn_collect off)
-and 64 bits.  Integer-valued rows below 2^11 have no second part and exact
-sums, so there both paths give the same tables bit for bit; on float rows the
-split path's error against 64 bits is no larger."""
+split into three bf16 parts, against the merging fp32 kernels (knn_collect off)
+and 64 bits.  Integer-valued rows have exact sums, so there both paths give
+the same tables bit for bit; on float rows the split path's error against 64
+bits is no larger."""
 import numpy as np
 import pytest
 
@@ -28,13 +28,13 @@ def _both(ctx, X, off, members, pr, M, metric="l2", running=None):
 
 
 @pytest.mark.parametrize("n,d,nb,probe,M", [
-    (3000, 161, 5, 1, 64), (2500, 256, 3, 0, 65), (4100, 288, 9, 2, 96), (1500, 500, 4, 1, 128),
-    (700, 1024, 3, 1, 5), (40, 300, 2, 0, 33), (1, 200, 1, 0, 8), (193, 960, 1, 0, 128), (2000, 992, 300, 3, 16),
+    (3000, 257, 5, 1, 64), (2500, 320, 3, 0, 65), (4100, 288, 9, 2, 96), (1500, 500, 4, 1, 128),
+    (700, 1024, 3, 1, 5), (40, 300, 2, 0, 33), (1, 270, 1, 0, 8), (193, 960, 1, 0, 128), (2000, 992, 300, 3, 16),
+    (66001, 288, 40, 1, 16),   # blocks of 256 queries, odd last ones
 ])
 def test_integer_rows_match_the_fp32_kernels(ctx, n, d, nb, probe, M):
     rng = np.random.default_rng(n + d)
     X = rng.integers(-60, 60, size=(n, d)).astype(np.float32)
-    X[:, 0] += 0.5 if d <= 256 else 0.0              # rows of at most 256 dimensions: not the int8 kernel's
     if n > 100:
         X[50:60] = X[40]                             # ties
     off, members, pr = _buckets(rng, n, nb, probe) if nb > 1 else (np.array([0, n]), np.arange(n, dtype=np.int32),
@@ -52,7 +52,43 @@ def test_integer_rows_match_the_fp32_kernels(ctx, n, d, nb, probe, M):
         np.testing.assert_array_equal(got[1], ref[1])
 
 
+@pytest.mark.parametrize("metric", ["l2", "ip"])
+def test_whole_numbers_beyond_two_parts(ctx, metric):
+    """One element of 2049..2895 per row: every sum is a whole number below
+    2^24, so exact in fp32; two rows of a kind lie at distance 0."""
+    rng = np.random.default_rng(4)
+    n, d = 4000, 300
+    X = np.zeros((n, d), np.float32)
+    X[np.arange(n), rng.integers(0, 5, size=n)] = rng.integers(2049, 2896, size=n)
+    X[n // 2:] = X[:n // 2]
+    got, ref = _both(ctx, X, np.array([0, n]), np.arange(n, dtype=np.int32), np.zeros((1, 0), np.int32), 8, metric)
+    np.testing.assert_array_equal(got[0], ref[0])
+    np.testing.assert_array_equal(got[1], ref[1])
+    assert metric == "ip" or (got[1][:, 0] == 0.0).all()
+
+
+@pytest.mark.parametrize("metric", ["l2", "ip"])
+@pytest.mark.parametrize("big,small", [(20, 0), (40, 0), (60, -50)])
+def test_rows_of_two_magnitudes(ctx, big, small, metric):
+    """Some rows with one huge coordinate, zero in all others: their inner
+    products are the small ones' alone, with all of their bits.  (2^110 apart:
+    more than the split rows hold, the fp32 kernel's launch.)"""
+    rng = np.random.default_rng(7)
+    n, d, rows = 1500, 300, 50
+    X = rng.integers(-20, 20, size=(n, d)).astype(np.float32) * np.float32(2.0 ** small)
+    X[:, :rows] = 0.0
+    X[np.arange(rows), np.arange(rows)] = 2.0 ** big
+    off, members, pr = _buckets(rng, n, 3, 1)
+    got, ref = _both(ctx, X, off, members, pr, 20, metric)
+    np.testing.assert_array_equal(got[0], ref[0])
+    np.testing.assert_array_equal(got[1], ref[1])
+
+
 def _rows(kind, rng, n, d):
+    if kind == "sparse":
+        X = np.zeros((n, d), np.float32)
+        X[np.arange(n)[:, None], np.argsort(rng.random((n, 12)), axis=1)[:, :3]] = rng.standard_normal((n, 3))
+        return X
     if kind == "mixture":
         return (rng.uniform(0, 1, (8, d))[rng.integers(0, 8, n)] + 0.1 * rng.standard_normal((n, d))).astype(np.float32)
     if kind == "latent":
@@ -62,8 +98,8 @@ def _rows(kind, rng, n, d):
     return (x / np.linalg.norm(x, axis=1, keepdims=True)).astype(np.float32)
 
 
-@pytest.mark.parametrize("d", [161, 256, 288, 512, 960, 1024])
-@pytest.mark.parametrize("kind,metric", [("mixture", "l2"), ("latent", "l2"), ("unit", "ip")])
+@pytest.mark.parametrize("d", [257, 288, 512, 960, 1024])
+@pytest.mark.parametrize("kind,metric", [("mixture", "l2"), ("latent", "l2"), ("unit", "ip"), ("sparse", "l2"), ("sparse", "ip")])
 def test_error_against_64_bits(ctx, kind, metric, d):
     rng = np.random.default_rng(d)
     n, M = 2000, 64
@@ -76,6 +112,7 @@ def test_error_against_64_bits(ctx, kind, metric, d):
     rms = []
     for ids, dist in _both(ctx, X, np.array([0, n]), np.arange(n, dtype=np.int32), np.zeros((1, 0), np.int32), M, metric):
         e = (dist - np.take_along_axis(full, ids.astype(np.int64), 1)) / np.take_along_axis(scale, ids.astype(np.int64), 1)
+        assert np.isfinite(e).all()
         rms.append(float(np.sqrt((e * e).mean())) * 2 ** 24)
     print(f"wide split d={d} {kind} {metric}: rms error {rms[0]:.3f} ulps, fp32 kernel {rms[1]:.3f}", flush=True)
     # the same sums in another order: 5 % for the sample (128,000 distances)

@@ -153,7 +153,13 @@ struct DevBuf {
     DevBuf() = default;
     DevBuf(const DevBuf&) = delete;
     DevBuf& operator=(const DevBuf&) = delete;
-    ~DevBuf() { if (p) (void)hipFree(p); }
+    ~DevBuf() { release(); }
+    void release()
+    {
+        if (p) (void)hipFree(p);
+        p = nullptr;
+        cap = 0;
+    }
     void* ensure(size_t bytes) {
         if (bytes <= cap) return p;
         if (p) GT_HIP(hipFree(p));
@@ -287,6 +293,9 @@ struct gt_ctx {
     uint64_t split_gen = 0;     // data_gen whose rows for the split W_XSPLIT / W_XSEXP hold (0: none)
     uint64_t split_order = 0;   // members_ver of their order (0: by row id)
     bool split_bad = false;     // some of them the inner product cannot take
+    bool split_live = false;    // a launch on them is being prepared
+    bool split_off = false;     // their memory was not to be had: the rest of this call runs without them
+    size_t mem_total = 0;       // device memory of this GPU
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     void* scratch = nullptr;    // this device's fixed scratch array (gt_optimize_noalloc), or null
     std::string scratch_err;    // why it is null
@@ -324,7 +333,23 @@ struct Ctx {
     gt_ctx* c;
     hipStream_t s;
     explicit Ctx(gt_ctx* cc) : c(cc), s(cc->stream) {}
-    template <typename T> T* ws(int slot, size_t n) { return c->ws[slot].as<T>(n); }
+    // a workspace; where memory has run out, at the price of the rows kept for the split
+    template <typename T> T* ws(int slot, size_t n) {
+        try {
+            return c->ws[slot].as<T>(n);
+        } catch (const Error& e) {
+            if (e.code != GT_ENOMEM || !release_split()) throw;
+        }
+        return c->ws[slot].as<T>(n);
+    }
+    bool release_split() {
+        (void)hipGetLastError();
+        if (c->split_live || c->ws[W_XSPLIT].cap + c->ws[W_QSPLIT].cap == 0) return false;
+        c->ws[W_XSPLIT].release();
+        c->ws[W_QSPLIT].release();
+        c->split_gen = 0;
+        return true;
+    }
     void sync() { GT_HIP(hipStreamSynchronize(s)); }
     void h2d(void* dst, const void* src, size_t bytes) {
         if (bytes) GT_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s));
@@ -510,7 +535,7 @@ static DevMatrix prepare(Ctx& c, int slot_x, int slot_raw, int slot_norms, const
     if (with_i8 && (dtype == GT_DTYPE_U8 || dtype == GT_DTYPE_I8) && Dp <= 256) {
         // integer rows: float copy, int8 copy and both norms in one pass
         if (!dev) {
-            void* raw = c.c->ws[slot_raw].ensure(static_cast<size_t>(N) * D * es);
+            void* raw = c.ws<uint8_t>(slot_raw, static_cast<size_t>(N) * D * es);
             c.upload(raw, X, static_cast<size_t>(N) * D * es);
             src = raw;
         }
@@ -532,7 +557,7 @@ static DevMatrix prepare(Ctx& c, int slot_x, int slot_raw, int slot_norms, const
         m.data = static_cast<const float*>(X);
     } else {
         if (!dev) {
-            void* raw = c.c->ws[slot_raw].ensure(static_cast<size_t>(N) * D * es);
+            void* raw = c.ws<uint8_t>(slot_raw, static_cast<size_t>(N) * D * es);
             c.upload(raw, X, static_cast<size_t>(N) * D * es);
             src = raw;
         }
@@ -1117,28 +1142,55 @@ static void sub_order_members(Ctx& c, const DevMatrix& X, const Buckets& b, int 
     ++c.c->members_ver;
 }
 
-// The rows of X in the scale and order that the collect kernel for split rows
-// takes (knn_wide_collect.hip), by position in the member list (null: by row
-// id), once per order; false where the copy is beyond 64 GiB, or it and the
-// launch's candidate slots would not leave half of the free device memory, or
-// the inner product meets a row that it needs the fp32 kernel for.
-static bool split_rows(Ctx& c, const DevMatrix& X, const int32_t* d_members, int64_t rows, int metric)
+// Room for a launch over split rows (knn_wide_collect.hip): the copy of the
+// rows, `slots` rows of candidates, and the queries' own copy (exact kNN).
+// Whether there is one follows from the sizes and the GPU's memory as built:
+// a quarter of it, and 64 GiB for the copy (`most`: the slots of a call's
+// largest launch, so that all launches of a call go the same way).  Only where
+// that much is not to be had, other programs holding it, does the call go on
+// with the fp32 kernels, whose keys are rounded otherwise.
+struct SplitUse {   // from the reservation to the launch: the copy is not given back
+    gt_ctx* c;
+    explicit SplitUse(gt_ctx* cc) : c(cc) {}
+    ~SplitUse() { c->split_live = false; }
+};
+static bool split_reserve(Ctx& c, const DevMatrix& X, int64_t slots, int64_t most, int64_t queries)
 {
-    const int64_t N = X.N;
-    const size_t need = split_copy_bytes(N, X.Dp), cand = static_cast<size_t>(rows + kQueriesPerWave) * kCollectCap * 8;
-    const size_t more = (c.c->ws[W_XSPLIT].cap < need ? need : 0) + (c.c->ws[W_CAND].cap < cand ? cand : 0);
-    if (need > size_t(16) << 32) return false;
-    if (more > 0) {
-        size_t fr = 0, total = 0;
-        GT_HIP(hipMemGetInfo(&fr, &total));
-        if (more > fr / 2) return false;
+    const size_t copy = split_copy_bytes(X.N, X.Dp), qcopy = queries > 0 ? split_copy_bytes(queries, X.Dp) : 0;
+    const size_t row = kCollectCap * sizeof(uint64_t);
+    if (c.c->split_off || copy > size_t(16) << 32 || copy + qcopy + static_cast<size_t>(most) * row > c.c->mem_total / 4)
+        return false;
+    try {
+        auto& ws = c.c->ws;
+        ws[W_XSPLIT].ensure(copy);
+        ws[W_XSEXP].as<int32_t>(static_cast<size_t>(X.N));
+        if (queries > 0) {
+            ws[W_QSPLIT].ensure(qcopy);
+            ws[W_QSEXP].as<int32_t>(static_cast<size_t>(queries));
+        }
+        ws[W_CAND].ensure(static_cast<size_t>(slots + kQueriesPerWave) * row);
+        ws[W_CANDCNT].as<int32_t>(static_cast<size_t>(slots));
+    } catch (const Error& e) {
+        if (e.code != GT_ENOMEM) throw;
+        (void)c.release_split();
+        c.c->split_off = true;
+        if (Trace().on) std::fprintf(stderr, "[gtann] no memory for split rows: fp32 kernels\n");
+        return false;
     }
-    float* xs = c.ws<float>(W_XSPLIT, need / 4);
-    int32_t* ex = c.ws<int32_t>(W_XSEXP, static_cast<size_t>(N));
-    unsigned int* bad = c.ws<unsigned int>(W_XSBAD, 1);
+    c.c->split_live = true;
+    return true;
+}
+
+// The rows of X in the scale and order that the kernel takes, by position in
+// the member list (null: by row id), once per order; false where the inner
+// product meets a row that it needs the fp32 kernel for.
+static bool split_rows(Ctx& c, const DevMatrix& X, const int32_t* d_members, int metric)
+{
     const uint64_t order = d_members ? c.c->members_ver : 0;
     if (c.c->split_gen != c.c->data_gen || c.c->split_order != order) {
-        launch_split_rows(X.data, X.norms, d_members, N, X.Dp, xs, ex, bad, c.s);
+        unsigned int* bad = c.ws<unsigned int>(W_XSBAD, 1);
+        launch_split_rows(X.data, X.norms, d_members, X.N, X.Dp, c.ws<float>(W_XSPLIT, 0), c.ws<int32_t>(W_XSEXP, 0), bad,
+                          c.s);
         c.c->split_gen = c.c->data_gen;
         c.c->split_order = order;
         c.c->split_bad = false;
@@ -1236,12 +1288,13 @@ static double bucketed_round(Ctx& c, const DevMatrix& X, const Buckets& b, int M
     // (Rows of 161 to 256 stay on the fp32 kernel: its one chain of sums has
     // errors of up to 4 ulps rms there, and more exact sums would change 1.7
     // to 2.1 % of a table's positions, near ties.)
-    const bool wide = c.c->dbg.knn_collect != 0 && !use_i8(X, X, metric) && X.Dp > 256 && M > 4 && M <= 128 &&
-                      split_rows(c, X, d_members, rows, metric);
-    const int qstep = wide ? wide_queries_per_block(rows) : kQueriesPerBlock;
     CopyTaskH* d_tasks = c.ws<CopyTaskH>(W_TASKS, tasks.size());
     c.h2d(d_tasks, tasks.data(), tasks.size() * sizeof(CopyTaskH));
     int32_t* d_pool = c.ws<int32_t>(W_POOL, static_cast<size_t>(std::max<int64_t>(total, 1)));
+    const SplitUse use(c.c);
+    const bool wide = c.c->dbg.knn_collect != 0 && !use_i8(X, X, metric) && X.Dp > 256 && M > 4 && M <= 128 &&
+                      split_reserve(c, X, rows, N, 0) && split_rows(c, X, d_members, metric);
+    const int qstep = wide ? wide_queries_per_block(rows) : kQueriesPerBlock;
     launch_copy_ranges(d_tasks, static_cast<int64_t>(tasks.size()), d_members, d_pool, c.s);
     int32_t* d_ppos = nullptr;   // wide: the pool entries' positions in the member list
     if (wide) {
@@ -1511,7 +1564,9 @@ static bool knn_exact_split(Ctx& c, const DevMatrix& X, const int32_t* d_q, int6
         const int64_t n = std::min(kBatch, nq - b0);
         slots = std::max(slots, slices(n, block(n)) * n);
     }
-    if (!split_rows(c, X, nullptr, slots, metric)) return false;
+    const int64_t batch = std::min(kBatch, nq);
+    const SplitUse use(c.c);
+    if (!split_reserve(c, X, slots, slots, d_q ? batch : 0) || !split_rows(c, X, nullptr, metric)) return false;
     const float* xs = c.ws<float>(W_XSPLIT, 0);
     const int32_t* ex = c.ws<int32_t>(W_XSEXP, 0);
     uint64_t* cand = c.ws<uint64_t>(W_CAND, static_cast<size_t>(slots + kQueriesPerWave) * kCollectCap);
@@ -1523,8 +1578,8 @@ static bool knn_exact_split(Ctx& c, const DevMatrix& X, const int32_t* d_q, int6
         const float* qs = xs;
         const int32_t* qex = ex;
         if (d_q) {
-            float* q = c.ws<float>(W_QSPLIT, split_copy_bytes(std::min(kBatch, nq), X.Dp) / 4);
-            int32_t* e = c.ws<int32_t>(W_QSEXP, static_cast<size_t>(std::min(kBatch, nq)));
+            float* q = c.ws<float>(W_QSPLIT, 0);
+            int32_t* e = c.ws<int32_t>(W_QSEXP, 0);
             launch_split_rows(X.data, X.norms, d_q + b0, n, X.Dp, q, e, c.ws<unsigned int>(W_XSBAD, 1), c.s);
             qs = q;
             qex = e;
@@ -2649,6 +2704,7 @@ static int guarded(gt_ctx* ctx, F&& f)
     try {
         GT_HIP(hipSetDevice(ctx->device));
         ctx->err.clear();
+        ctx->split_off = false;
         f();
         return GT_OK;
     } catch (const Error& e) {
@@ -2738,6 +2794,11 @@ int gt_create(int device, gt_ctx** out)
         delete c;
         return GT_EDEVICE;
     }
+    size_t free_now = 0;
+    if (hipMemGetInfo(&free_now, &c->mem_total) != hipSuccess) {
+        delete c;
+        return GT_EDEVICE;
+    }
     // this device's scratch address (looked up once per device); a failure
     // only disables gt_optimize_noalloc
     c->scratch = scratch_for_device(device, c->scratch_err);
@@ -2750,11 +2811,7 @@ void gt_destroy(gt_ctx* ctx)
     if (!ctx) return;
     (void)hipSetDevice(ctx->device);
     (void)hipStreamSynchronize(ctx->stream);
-    for (auto& b : ctx->ws) {
-        if (b.p) (void)hipFree(b.p);
-        b.p = nullptr;
-        b.cap = 0;
-    }
+    for (auto& b : ctx->ws) b.release();
     for (auto& pb : ctx->pinned) pb.release();
     ctx->pin_stage.release();
     for (hipEvent_t e : ctx->stage_ev)

@@ -40,6 +40,13 @@ enum { GT_METRIC_L2 = 0, GT_METRIC_IP = 1 };
 enum { GT_SEED_AUTO = 0, GT_SEED_KMEANS_PAR = 1, GT_SEED_UNIFORM = 2 };
 
 /* Context owning a device, a stream and reusable workspaces.
+ * Among them, for exact kNN and for bucketed kNN and builds of float rows
+ * beyond 256 dimensions: the rows in another order (4 bytes per padded
+ * element) and the launch's candidates.  Whether a call takes that path
+ * follows from its sizes and the GPU's memory as built (both within a quarter
+ * of it), never from what is free; where that much is held by others, the
+ * call runs on kernels that round distances otherwise (near ties may change
+ * places).  The copy is given back when another call needs its room.
  * Replaces the GpuResidentKnn constructor/destructor
  * (src/bucket.cu:5216-5241, :5650) and the cuVS raft::resources handle. */
 int gt_create(int device, gt_ctx** out);

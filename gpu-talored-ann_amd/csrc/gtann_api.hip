@@ -1540,18 +1540,26 @@ static double bucketed_round(Ctx& c, const DevMatrix& X, const Buckets& b, int M
 // two per CU in all), then each query's top k over its slices' candidates;
 // kBatch queries at a time (as many as make 512 blocks by themselves), which
 // bounds the candidate slots to 256 MiB.
-// false: not this path's -- integer rows, short lists, few queries (the split
-// copy costs a pass over the rows, which below kMinQueries queries takes
-// longer than it saves), and rows of 129 to 256 dimensions, where the fp32
-// kernel's one chain of sums rounds most: it orders 1.1 to 1.6 % of a long
-// list's positions, near ties, otherwise than more exact sums do (0.85 % at
-// 128, 0.2 % beyond 256), and callers keep the lists they have.
+// false: not this path's --
+//  * integer rows, which are exact on the int8 matrix cores;
+//  * lists of up to 4: the fp32 kernels hold those in registers (1-NN of 512
+//    in 200,003 x 100: 0.66 ms here, 0.50 there; 10-NN 0.70 and 1.06);
+//  * fewer than kMinRows rows: short calls on either path (10-NN in 1,000 x
+//    100: of one query 0.20 and 0.18 ms, of 1,000 0.23 and 0.35; in 4,096 x
+//    100: 0.29 and 0.45, 0.31 and 0.75);
+//  * rows of 129 to 256 dimensions, where the fp32 kernel's one chain of sums
+//    rounds most: it orders 1.1 to 1.6 % of a long list's positions, near
+//    ties, otherwise than more exact sums do (0.85 % at 128, 0.2 % beyond
+//    256), and callers keep the lists they have.
+// The number of queries is not asked for: a query's list is the same in any
+// batch.  (One query in 1,000,003 x 100, k 10: 1.24 ms here, 2.03 there; in
+// 20,000 x 32: 0.21 and 0.20.)
 static bool knn_exact_split(Ctx& c, const DevMatrix& X, const int32_t* d_q, int64_t nq, int k, int metric,
                             int32_t* out_ids, float* out_d)
 {
-    constexpr int64_t kMinQueries = 256, kMinRows = 4096, kSliceRows = 2048, kBatch = 512 * 256;
-    if (c.c->dbg.knn_collect == 0 || use_i8(X, X, metric) || k <= 4 || k > 128 || nq < kMinQueries ||
-        X.N < kMinRows || (X.Dp > 128 && X.Dp <= 256))
+    constexpr int64_t kMinRows = 4096, kSliceRows = 2048, kBatch = 512 * 256;
+    if (c.c->dbg.knn_collect == 0 || use_i8(X, X, metric) || k <= 4 || k > 128 || X.N < kMinRows ||
+        (X.Dp > 128 && X.Dp <= 256))
         return false;
     const int64_t by_pool = X.N / kSliceRows;
     // slices of a batch of n queries in blocks of qpb

@@ -59,7 +59,11 @@ const char* gt_version(void);
 
 /* Exact kNN of the query rows `queries[0..nq)` (all N rows when queries is
  * NULL, then nq must be N) against all N rows, self excluded.
- * ids/dists: nq x k.  Replaces bd/build_knn.py:98-149 (build_exact_knn). */
+ * ids/dists: nq x k.  A query's list does not depend on the other queries of
+ * the call.  Float rows' distances are rounded sums, and their last bits may
+ * differ between lists of up to 4 and longer ones, and from the bucketed
+ * calls': near ties may change places.
+ * Replaces bd/build_knn.py:98-149 (build_exact_knn). */
 int gt_knn_exact(gt_ctx* ctx, const void* X, int64_t N, int32_t D, int dtype, int metric,
                  const int64_t* queries, int64_t nq, int32_t k, int32_t* ids, float* dists);
 

@@ -44,6 +44,19 @@ def test_slices_match_the_fp32_kernels(ctx, n, d, nq, k, distinct):
         _same(ctx, X, k, q, metric)
 
 
+@pytest.mark.parametrize("metric", ["l2", "ip"])
+@pytest.mark.parametrize("d", [33, 128, 300])
+def test_lists_do_not_depend_on_the_batch(ctx, d, metric):
+    rng = np.random.default_rng(d)
+    X = rng.standard_normal((20011, d)).astype(np.float32)
+    q = rng.permutation(20011)[:3000]
+    ids, dist = ctx.knn_exact(X, 20, queries=q, metric=metric)
+    for nq in (1, 2, 33, 128, 255, 256, 700):
+        i, v = ctx.knn_exact(X, 20, queries=q[:nq], metric=metric)
+        np.testing.assert_array_equal(i, ids[:nq])
+        np.testing.assert_array_equal(v.view(np.uint32), dist[:nq].view(np.uint32))
+
+
 @pytest.mark.parametrize("d", [1, 100, 300])
 def test_whole_numbers_beyond_two_parts(ctx, d):
     """One element of 2049..2895 per row: every sum is a whole number below

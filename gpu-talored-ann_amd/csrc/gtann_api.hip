@@ -1182,15 +1182,20 @@ static bool split_reserve(Ctx& c, const DevMatrix& X, int64_t slots, int64_t mos
 }
 
 // The rows of X in the scale and order that the kernel takes, by position in
-// the member list (null: by row id), once per order; false where the inner
-// product meets a row that it needs the fp32 kernel for.
-static bool split_rows(Ctx& c, const DevMatrix& X, const int32_t* d_members, int metric)
+// the member list (null: by row id), once per order (*t: plus the seconds it
+// took); false where the inner product meets a row that it needs the fp32
+// kernel for.
+static bool split_rows(Ctx& c, const DevMatrix& X, const int32_t* d_members, int metric, double* t = nullptr)
 {
     const uint64_t order = d_members ? c.c->members_ver : 0;
     if (c.c->split_gen != c.c->data_gen || c.c->split_order != order) {
         unsigned int* bad = c.ws<unsigned int>(W_XSBAD, 1);
-        launch_split_rows(X.data, X.norms, d_members, X.N, X.Dp, c.ws<float>(W_XSPLIT, 0), c.ws<int32_t>(W_XSEXP, 0), bad,
-                          c.s);
+        auto copy = [&] {
+            launch_split_rows(X.data, X.norms, d_members, X.N, X.Dp, c.ws<float>(W_XSPLIT, 0), c.ws<int32_t>(W_XSEXP, 0),
+                              bad, c.s);
+        };
+        if (t) *t += c.timed(copy);
+        else copy();
         c.c->split_gen = c.c->data_gen;
         c.c->split_order = order;
         c.c->split_bad = false;
@@ -1292,15 +1297,13 @@ static double bucketed_round(Ctx& c, const DevMatrix& X, const Buckets& b, int M
     c.h2d(d_tasks, tasks.data(), tasks.size() * sizeof(CopyTaskH));
     int32_t* d_pool = c.ws<int32_t>(W_POOL, static_cast<size_t>(std::max<int64_t>(total, 1)));
     const SplitUse use(c.c);
+    double t = 0.0;   // device seconds
     const bool wide = c.c->dbg.knn_collect != 0 && !use_i8(X, X, metric) && X.Dp > 256 && M > 4 && M <= 128 &&
-                      split_reserve(c, X, rows, N, 0) && split_rows(c, X, d_members, metric);
+                      split_reserve(c, X, rows, N, 0) && split_rows(c, X, d_members, metric, &t);
     const int qstep = wide ? wide_queries_per_block(rows) : kQueriesPerBlock;
     launch_copy_ranges(d_tasks, static_cast<int64_t>(tasks.size()), d_members, d_pool, c.s);
-    int32_t* d_ppos = nullptr;   // wide: the pool entries' positions in the member list
-    if (wide) {
-        d_ppos = c.ws<int32_t>(W_XSPOS, static_cast<size_t>(std::max<int64_t>(total, 1)));
-        launch_copy_ranges(d_tasks, static_cast<int64_t>(tasks.size()), nullptr, d_ppos, c.s);
-    }
+    // wide: the pool entries' positions in the member list
+    int32_t* d_ppos = wide ? c.ws<int32_t>(W_XSPOS, static_cast<size_t>(std::max<int64_t>(total, 1))) : nullptr;
 
     std::vector<std::vector<WorkItem>> groups(static_cast<size_t>(C));
     int64_t mp = 0, mb = 0;
@@ -1349,8 +1352,8 @@ static double bucketed_round(Ctx& c, const DevMatrix& X, const Buckets& b, int M
     a.seed_ld = M;
     a.out_ids = out_ids;
     a.out_d = out_d;
-    // lists of at most 64 keys on int8 rows: collect + select (every point
-    // is the query of exactly one work item, so rows = N)
+    // collect + select where it applies (every point is the query of exactly
+    // one work item, so rows = N)
     const bool collect = wide || (c.c->dbg.knn_collect != 0 && knn_collect_supported(a));
     if (collect) {
         // (+ one wave's rows of slack: the selection reads whole groups of
@@ -1461,7 +1464,7 @@ static double bucketed_round(Ctx& c, const DevMatrix& X, const Buckets& b, int M
         a.chr = c.ws<float>(W_CHR, static_cast<size_t>(std::max<int64_t>(nchunk, 1)));
     }
     const double done_before = c.c->knn_pairs_done;
-    const double t = c.timed([&] {
+    t += c.timed([&] {
         if (prune)
             launch_chunk_bounds(X.data8, X.Dp8, d_pool, d_chcnt, nchunk, const_cast<int8_t*>(a.ch8),
                                 const_cast<float*>(a.chn), const_cast<float*>(a.chr), c.s);
@@ -1481,6 +1484,7 @@ static double bucketed_round(Ctx& c, const DevMatrix& X, const Buckets& b, int M
         if (wide) {
             const float* xs = c.ws<float>(W_XSPLIT, 0);
             const int32_t* ex = c.ws<int32_t>(W_XSEXP, 0);
+            launch_copy_ranges(d_tasks, static_cast<int64_t>(tasks.size()), nullptr, d_ppos, c.s);
             launch_wide_collect(a, qstep, xs, ex, xs, ex, d_ppos, c.s);
             launch_collect_select(a, rows, c.s);
         } else if (collect) {

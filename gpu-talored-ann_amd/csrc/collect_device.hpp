@@ -1,6 +1,6 @@
 // collect_device.hpp -- device pieces shared by the collect kernels
 // (knn_collect.hip: int8 and fp32 rows in LDS tiles; knn_wide_collect.hip:
-// rows split into two fp16 parts).
+// rows split into three bf16 parts).
 #pragma once
 
 #include "knn_device.hpp"
@@ -44,32 +44,14 @@ __device__ __forceinline__ bool key_passes(float d, int32_t id, const CollectSta
 }
 
 // Drops the largest of query q's cnt (> M) keys: its slots keep the M smallest
-// and at most kCompactSlack more, and the largest distance kept becomes its
-// threshold.  The distance is found by bisection over the ordered bits of the
+// and at most kCompactSlack more (up to kCollectCap - 64 in all where more tie
+// at the last distance), and the largest distance kept becomes its threshold.  The distance is found by bisection over the ordered bits of the
 // keys' distances (about 7 steps of a compare and a bit count per 64 keys; the
 // exact M-th key takes 64 such steps over both words, 1,100 instructions, and
 // made up most of the wide kernel's vector work).  Only where more keys tie
 // there than the slots can spare is it the M-th key in (distance, id) order.
 // Called by all 64 lanes; q is uniform.
 constexpr int kCompactSlack = 16;
-
-template <bool MAX>
-__device__ __forceinline__ uint32_t wave_extreme_u32(uint32_t x)
-{
-    auto f = [](uint32_t a, uint32_t b) { return MAX ? max(a, b) : min(a, b); };
-    auto dpp = [](uint32_t v, auto ctrl, auto rows) {
-        return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(static_cast<int>(v), static_cast<int>(v), decltype(ctrl)::value,
-                                                                 decltype(rows)::value, 0xf, false));
-    };
-    using std::integral_constant;
-    x = f(x, dpp(x, integral_constant<int, 0x111>{}, integral_constant<int, 0xf>{}));   // row_shr:1, 2, 4, 8
-    x = f(x, dpp(x, integral_constant<int, 0x112>{}, integral_constant<int, 0xf>{}));
-    x = f(x, dpp(x, integral_constant<int, 0x114>{}, integral_constant<int, 0xf>{}));
-    x = f(x, dpp(x, integral_constant<int, 0x118>{}, integral_constant<int, 0xf>{}));
-    x = f(x, dpp(x, integral_constant<int, 0x142>{}, integral_constant<int, 0xa>{}));   // row_bcast:15, 31
-    x = f(x, dpp(x, integral_constant<int, 0x143>{}, integral_constant<int, 0xc>{}));
-    return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(x), 63));
-}
 
 __device__ __forceinline__ void collect_compact(const KnnArgs& a, int lane, int q, CollectState& st)
 {

@@ -240,4 +240,27 @@ __device__ __forceinline__ uint64_t shfl_xor_u64(uint64_t v, int m)
     return (static_cast<uint64_t>(hi) << 32) | lo;
 }
 
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint32_t dpp_u32(uint32_t x)
+{
+    return static_cast<uint32_t>(
+        __builtin_amdgcn_update_dpp(static_cast<int>(x), static_cast<int>(x), CTRL, ROWS, 0xf, false));
+}
+
+// Maximum / minimum over the 64 lanes (uniform): row shifts by 1, 2, 4 and 8
+// reduce each row of 16 lanes into its last lane, the two broadcasts carry the
+// rows into lane 63; a lane without a source keeps its own value.
+template <bool MAX>
+__device__ __forceinline__ uint32_t wave_extreme_u32(uint32_t x)
+{
+    auto f = [](uint32_t a, uint32_t b) { return MAX ? max(a, b) : min(a, b); };
+    x = f(x, dpp_u32<0x111, 0xf>(x));
+    x = f(x, dpp_u32<0x112, 0xf>(x));
+    x = f(x, dpp_u32<0x114, 0xf>(x));
+    x = f(x, dpp_u32<0x118, 0xf>(x));
+    x = f(x, dpp_u32<0x142, 0xa>(x));
+    x = f(x, dpp_u32<0x143, 0xc>(x));
+    return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(x), 63));
+}
+
 }  // namespace gtann

@@ -75,41 +75,18 @@ __device__ __forceinline__ uint32_t readlane_u(uint32_t v, int l)
     return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), l));
 }
 
-template <int CTRL, int ROWS>
-__device__ __forceinline__ uint32_t dpp_u(uint32_t x)
-{
-    return static_cast<uint32_t>(
-        __builtin_amdgcn_update_dpp(static_cast<int>(x), static_cast<int>(x), CTRL, ROWS, 0xf, false));
-}
-
-// Maximum / minimum over the 64 lanes (uniform): row shifts by 1, 2, 4 and 8
-// reduce each row of 16 lanes into its last lane, the two broadcasts carry the
-// rows into lane 63; a lane without a source keeps its own value.
-template <bool MAX>
-__device__ __forceinline__ uint32_t wave_extreme(uint32_t x)
-{
-    auto f = [](uint32_t a, uint32_t b) { return MAX ? max(a, b) : min(a, b); };
-    x = f(x, dpp_u<0x111, 0xf>(x));
-    x = f(x, dpp_u<0x112, 0xf>(x));
-    x = f(x, dpp_u<0x114, 0xf>(x));
-    x = f(x, dpp_u<0x118, 0xf>(x));
-    x = f(x, dpp_u<0x142, 0xa>(x));
-    x = f(x, dpp_u<0x143, 0xc>(x));
-    return readlane_u(x, 63);
-}
-
 // The smallest of the lanes' 64-bit keys (uniform): the high words first, the
 // low words only among the lanes that tie there.
 __device__ __forceinline__ uint64_t wave_min_u64(uint64_t k)
 {
     const uint32_t hi = static_cast<uint32_t>(k >> 32);
-    const uint32_t mh = wave_extreme<false>(hi);
+    const uint32_t mh = wave_extreme_u32<false>(hi);
     const uint64_t tie = __ballot(hi == mh);
     uint32_t ml;
     if ((tie & (tie - 1)) == 0)
         ml = readlane_u(static_cast<uint32_t>(k), __ffsll(static_cast<unsigned long long>(tie)) - 1);
     else
-        ml = wave_extreme<false>(hi == mh ? static_cast<uint32_t>(k) : 0xFFFFFFFFu);
+        ml = wave_extreme_u32<false>(hi == mh ? static_cast<uint32_t>(k) : 0xFFFFFFFFu);
     return (static_cast<uint64_t>(mh) << 32) | ml;
 }
 
@@ -289,7 +266,7 @@ struct BestList {
                 first = k[r] > m ? r : first;
                 m = max(m, k[r]);
             }
-            key = wave_extreme<true>(m);
+            key = wave_extreme_u32<true>(m);
             const int l = __ffsll(static_cast<unsigned long long>(__ballot(m == key))) - 1;
             slot = R * l + (R > 1 ? __builtin_amdgcn_readlane(first, l) : 0);
         } else {
@@ -298,8 +275,8 @@ struct BestList {
                 first = (x > m || i == lane) ? i : first;
                 m = max(m, x);
             }
-            key = wave_extreme<true>(m);
-            slot = static_cast<int>(wave_extreme<false>(lane < ef && m == key ? static_cast<uint32_t>(first) : 0xFFFFFFFFu));
+            key = wave_extreme_u32<true>(m);
+            slot = static_cast<int>(wave_extreme_u32<false>(lane < ef && m == key ? static_cast<uint32_t>(first) : 0xFFFFFFFFu));
         }
     }
 };

@@ -321,13 +321,17 @@ static_assert(W_COUNT_ <= 128, "workspace slots");
 // memcpy over the host pool's threads
 static void parallel_copy(void* dst, const void* src, size_t bytes);
 
-// Pageable arrays from kStageMin bytes on go through two pinned halves of
-// kStageChunk bytes: the threads copy one while the DMA moves the other.  Left
-// to the runtime the transfer pins or copies the pages from one thread, and a
-// fresh output array is faulted in one page after another (gt_optimize of a
-// 51 MB table to a 26 MB graph: 4.3 -> 2.7 ms).  Smaller arrays take the
-// runtime's path: a chunk's hand-over to the threads would not pay.
-constexpr size_t kStageMin = size_t(8) << 20, kStageChunk = size_t(4) << 20;
+// Large pageable arrays go through two pinned halves of kStageChunk bytes: the
+// threads copy one while the DMA moves the other.  Left to the runtime the
+// transfer pins or copies the pages from one thread, and a fresh output array
+// is faulted in one page after another (gt_optimize of a 51 MB table to a
+// 26 MB graph: 4.3 -> 2.7 ms).  The limits are where waking the threads starts
+// to pay (whole calls, both routes in turn).  Results, two arrays of gt_knn_exact,
+// touched before / fresh: 1 MiB 0.46 and 0.43 / 0.80 and 0.90 ms (staged and
+// runtime), 2 MiB 0.55 and 0.58 / 1.25 and 1.55, 8 MiB 2.0 and 2.5 / 4.7 and
+// 6.4.  Inputs, rows of gt_knn_exact: 8 MiB 0.57 and 0.47, 24 MiB 1.01 and
+// 0.97, 32 MiB 1.29 and 1.36.
+constexpr size_t kUploadMin = size_t(32) << 20, kDownloadMin = size_t(2) << 20, kStageChunk = size_t(4) << 20;
 
 struct Ctx {
     gt_ctx* c;
@@ -369,10 +373,9 @@ struct Ctx {
             return nullptr;
         }
     }
-    static bool stageable(const void* host, size_t bytes) { return bytes >= kStageMin && !is_pinned_ptr(host); }
     // a caller's host array to the device; the array has been read when it returns, as with h2d of pageable memory
     void upload(void* dst, const void* src, size_t bytes) {
-        unsigned char* st = stageable(src, bytes) ? stage() : nullptr;
+        unsigned char* st = bytes >= kUploadMin && !is_pinned_ptr(src) ? stage() : nullptr;
         if (!st) return h2d(dst, src, bytes);
         for (size_t at = 0, i = 0; at < bytes; at += kStageChunk, ++i) {
             const size_t n = std::min(kStageChunk, bytes - at);
@@ -385,7 +388,7 @@ struct Ctx {
     }
     // device results to a caller's host array; complete when it returns if they are staged, else after a sync
     void download(void* dst, const void* src, size_t bytes) {
-        unsigned char* st = stageable(dst, bytes) ? stage() : nullptr;
+        unsigned char* st = bytes >= kDownloadMin && !is_pinned_ptr(dst) ? stage() : nullptr;
         if (!st) return d2h(dst, src, bytes);
         const size_t chunks = (bytes + kStageChunk - 1) / kStageChunk;
         auto size = [&](size_t i) { return std::min(kStageChunk, bytes - i * kStageChunk); };

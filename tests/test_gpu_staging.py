@@ -1,5 +1,6 @@
-"""Pageable arrays of 8 MiB and more go through two pinned halves of 4 MiB:
-the same results as device tensors, whatever the last chunk's length."""
+"""Pageable inputs of 32 MiB and more and results of 2 MiB and more go through
+two pinned halves of 4 MiB: the same results as device tensors, whatever the
+last chunk's length."""
 import numpy as np
 import pytest
 
@@ -8,8 +9,11 @@ import gt_oracle as O
 pytestmark = pytest.mark.gpu
 
 
-# rows of 4 bytes x d: below the limit, at it, one element past it and past a chunk, odd chunk counts
-@pytest.mark.parametrize("n,d,k", [(16383, 128, 5), (16384, 128, 128), (16391, 131, 127), (24577, 128, 86), (70001, 61, 33)])
+# rows of 4 bytes x d and results of 4 bytes x k: below the limits, at them, one element past them and past a chunk,
+# odd chunk counts
+@pytest.mark.parametrize("n,d,k", [(16383, 128, 5), (16384, 128, 128), (16391, 131, 127), (24577, 128, 86), (70001, 61, 33),
+                                   (65535, 128, 8), (65536, 128, 8), (65543, 131, 9), (98305, 129, 5), (8192, 64, 64),
+                                   (8191, 64, 64)])
 def test_host_arrays_match_device_tensors(ctx, n, d, k):
     import torch
     X = np.random.default_rng(n).integers(0, 50, size=(n, d)).astype(np.float32)

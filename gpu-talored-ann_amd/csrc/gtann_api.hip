@@ -295,6 +295,7 @@ struct gt_ctx {
     bool split_bad = false;     // some of them the inner product cannot take
     bool split_live = false;    // a launch on them is being prepared
     bool split_off = false;     // their memory was not to be had: the rest of this call runs without them
+    int split_pays = -1;        // this call's first bucketing: its buckets are large enough for them (-1: none yet)
     size_t mem_total = 0;       // device memory of this GPU
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     void* scratch = nullptr;    // this device's fixed scratch array (gt_optimize_noalloc), or null
@@ -1292,16 +1293,32 @@ static double bucketed_round(Ctx& c, const DevMatrix& X, const Buckets& b, int M
     const bool sub_ordered = own && !compact && c.c->dbg.sub_order != 0 && (!seed_d || want_prune || want_screen);
     if (sub_ordered) sub_order_members(c, X, b, metric, d_members);
     // fp32 rows longer than 256: collect on the bf16 matrix cores over rows
-    // split in three, 256 or 128 queries per block (lists of 5..128 keys).
+    // split in three, 256 or 128 queries per block (lists of 5..128 keys),
+    // where a point's bucket holds kSplitBucket rows or more on average: below
+    // that the copy and the candidates' passes cost more than the matrix cores
+    // save, and half-filled blocks more (own bucket and one probed, M 8, over a
+    // running table, times of the fp32 kernel's: 200,000 x 960 in buckets of
+    // 100 1.6, of 300 1.08, of 500 0.82, of 1,000 0.76; 50,000 x 960 in buckets
+    // of 300 1.27, of 500 0.79).  All passes of a call go by its first
+    // bucketing.
     // (Rows of 161 to 256 stay on the fp32 kernel: its one chain of sums has
     // errors of up to 4 ulps rms there, and more exact sums would change 1.7
     // to 2.1 % of a table's positions, near ties.)
     CopyTaskH* d_tasks = c.ws<CopyTaskH>(W_TASKS, tasks.size());
     c.h2d(d_tasks, tasks.data(), tasks.size() * sizeof(CopyTaskH));
     int32_t* d_pool = c.ws<int32_t>(W_POOL, static_cast<size_t>(std::max<int64_t>(total, 1)));
+    constexpr double kSplitBucket = 400.0;
+    if (c.c->split_pays < 0) {
+        double sq = 0.0;
+        for (int64_t bb = 0; bb < C; ++bb) {
+            const double n = static_cast<double>(b.offsets[static_cast<size_t>(bb + 1)] - b.offsets[static_cast<size_t>(bb)]);
+            sq += n * n;
+        }
+        c.c->split_pays = sq >= kSplitBucket * static_cast<double>(N) ? 1 : 0;
+    }
     const SplitUse use(c.c);
     double t = 0.0;   // device seconds
-    const bool wide = c.c->dbg.knn_collect != 0 && !use_i8(X, X, metric) && X.Dp > 256 && M > 4 && M <= 128 &&
+    const bool wide = (c.c->dbg.knn_collect == 2 || (c.c->dbg.knn_collect == 1 && c.c->split_pays)) && !use_i8(X, X, metric) && X.Dp > 256 && M > 4 && M <= 128 &&
                       split_reserve(c, X, rows, N, 0) && split_rows(c, X, d_members, metric, &t);
     const int qstep = wide ? wide_queries_per_block(rows) : kQueriesPerBlock;
     launch_copy_ranges(d_tasks, static_cast<int64_t>(tasks.size()), d_members, d_pool, c.s);
@@ -2720,6 +2737,7 @@ static int guarded(gt_ctx* ctx, F&& f)
         GT_HIP(hipSetDevice(ctx->device));
         ctx->err.clear();
         ctx->split_off = false;
+        ctx->split_pays = -1;
         f();
         return GT_OK;
     } catch (const Error& e) {

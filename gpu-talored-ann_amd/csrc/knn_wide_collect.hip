@@ -35,8 +35,8 @@
 // cores are busy: a block is 8 waves with 256 queries (32 per wave, read from
 // L2 chunk by chunk) against 192 pool rows at a time (32-dimension chunks
 // double-buffered in LDS, shared by the waves; 6 accumulator tiles of 32 x 32
-// per wave).  Launches with fewer blocks than the chip has CUs take 4 waves
-// and 128 queries.  A copy of the three parts, 6 bytes per element, was
+// per wave).  Short launches take 4 waves and 128 queries
+// (wide_queries_per_block).  A copy of the three parts, 6 bytes per element, was
 // slower: bucketed pass below 13.0 ms, build 187.
 // What bounds it (bucketed pass over 100,003 x 960, 25 buckets, one probe, M
 // 96; counters): where a CU has a block, its matrix cores are busy 57 % of the
@@ -613,9 +613,12 @@ void launch_split_select(const uint64_t* cand, const int32_t* cnt, int64_t nq, i
     GT_HIP(hipGetLastError());
 }
 
-// Queries per block of a launch over n_queries queries: 256 (8 waves) where
-// that gives every CU a block, else 128.
-int wide_queries_per_block(int64_t n_queries) { return n_queries >= int64_t(256) * 256 ? 256 : 128; }
+// Queries per block of a launch over n_queries queries: 128 (4 waves) where
+// those blocks, of which a CU holds one, make no more than one round, else 256
+// (8 waves).  Bucketed passes of 960 dimensions, buckets of 1,000, 128 and 256
+// queries per block: 32,000 rows 1.58 and 1.77 ms, 34,000 rows 2.75 and 1.84,
+// 60,000 rows 2.83 and 2.25.
+int wide_queries_per_block(int64_t n_queries) { return n_queries > int64_t(128) * 256 ? 256 : 128; }
 
 // Xs, ex: the split rows by position; p_pos: the position of every pool-list
 // entry (null: itself).  Qs, qex: the split queries, query i (its place in

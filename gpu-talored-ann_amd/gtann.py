@@ -287,8 +287,10 @@ class Context:
             raise GtannError(rc, f"{what}: {msg.decode() if msg else ''}")
 
     def set_debug(self, **opts):
-        """Path selection (gt_set_debug): every choice gives the same results.
-        Keywords: knn_collect (bool), revmerge_path ('auto'|'rv'|'binned'|'csr'|'rv2'),
+        """Path selection (gt_set_debug): every choice gives the same results,
+        but for the rounding of float rows' distances, which knn_collect
+        changes.  Keywords: knn_collect (0 merging kernels, 1, 2 split rows in
+        small buckets too), revmerge_path ('auto'|'rv'|'binned'|'csr'|'rv2'),
         sub_order (bool), lloyd_host_csr (bool), prune_flat_rows (bool),
         knn_stats (bool), knn_prune (bool), bucket_host_csr (bool),
         knn_resident (bool), knn_window (even tiles, 0 = by size),

@@ -21,7 +21,8 @@ def _buckets(rng, n, nb, probe):
 
 
 def _both(ctx, X, off, members, pr, M, metric="l2", running=None):
-    got = ctx.knn_bucketed(X, off, members, pr, M, metric=metric, running=running)
+    with debug_opts(ctx, knn_collect=2):               # buckets of any size
+        got = ctx.knn_bucketed(X, off, members, pr, M, metric=metric, running=running)
     with debug_opts(ctx, knn_collect=False):
         ref = ctx.knn_bucketed(X, off, members, pr, M, metric=metric, running=running)
     return got, ref
@@ -30,7 +31,7 @@ def _both(ctx, X, off, members, pr, M, metric="l2", running=None):
 @pytest.mark.parametrize("n,d,nb,probe,M", [
     (3000, 257, 5, 1, 64), (2500, 320, 3, 0, 65), (4100, 288, 9, 2, 96), (1500, 500, 4, 1, 128),
     (700, 1024, 3, 1, 5), (40, 300, 2, 0, 33), (1, 270, 1, 0, 8), (193, 960, 1, 0, 128), (2000, 992, 300, 3, 16),
-    (66001, 288, 40, 1, 16),   # blocks of 256 queries, odd last ones
+    (32769, 288, 20, 1, 16),   # blocks of 256 queries, odd last ones
 ])
 def test_integer_rows_match_the_fp32_kernels(ctx, n, d, nb, probe, M):
     rng = np.random.default_rng(n + d)
@@ -153,6 +154,21 @@ def test_small_scales(ctx, metric):
     got, ref = _both(ctx, X, off, members, pr, M, metric)
     np.testing.assert_array_equal(got[0], ref[0])
     np.testing.assert_array_equal(got[1], ref[1])
+
+
+@pytest.mark.parametrize("size", [40, 200, 350, 500, 1000])
+def test_small_buckets_stay_on_the_fp32_kernel(ctx, size):
+    """Buckets below 400 rows: the fp32 kernel's table; from there on the one over split rows."""
+    X = _rows("mixture", np.random.default_rng(size), 3000, 300)
+    nb = 3000 // size
+    off = np.linspace(0, 3000, nb + 1).astype(np.int64)
+    args = (X, off, np.arange(3000, dtype=np.int32), np.zeros((nb, 0), np.int32), 32)
+    split, fp32 = _both(ctx, *args)
+    got = ctx.knn_bucketed(*args)
+    assert (split[1].view(np.uint32) != fp32[1].view(np.uint32)).any()
+    want = fp32 if 3000 / nb < 400 else split
+    np.testing.assert_array_equal(got[0], want[0])
+    np.testing.assert_array_equal(got[1].view(np.uint32), want[1].view(np.uint32))
 
 
 def test_out_of_core_build(ctx):

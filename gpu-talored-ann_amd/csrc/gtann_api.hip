@@ -74,6 +74,7 @@ void launch_negate(float* d, int64_t n, hipStream_t s);
 void launch_graph_search(const SearchArgs& a, int dtype, int64_t grid, hipStream_t s);
 void launch_search_totals_init(SearchTotals* t, hipStream_t s);
 size_t search_query_lds(const SearchArgs& a, int esz);
+bool search_lane_rows(int64_t queries, int D, int degree, bool floats);
 void launch_invert_perm(const uint32_t* inv, int64_t N, uint32_t* perm, uint32_t* hits, int* err, hipStream_t s);
 void launch_permute_rows(const void* in, const uint32_t* inv, int64_t N, int64_t row_bytes, void* out, hipStream_t s);
 void launch_remap_table(const int32_t* ids, const uint32_t* inv, const uint32_t* perm, int64_t N, int M, int32_t* out,
@@ -3044,22 +3045,37 @@ int gt_search(gt_ctx* ctx, const void* X, int64_t N, int32_t D, int dtype, const
                 return static_cast<size_t>(a.CC) * 8 + static_cast<size_t>(a.efr) * 8 +
                            static_cast<size_t>(pad_dim(D)) * 4 + static_cast<size_t>(H) * 4 <= 65536;
             };
+            a.lane_rows = search_lane_rows(nq, D, degree, rows_dtype == GT_DTYPE_F32) ? 1 : 0;
             // by itself: room for 0.9 degree x ef points at 13/16 full (S2's
             // queries visit 0.76 of degree x ef at ef 200, 0.9 at ef 64 on
             // average), more where the queries leave LDS unused (a query
             // that outgrows its table costs its time twice), unless that
             // takes more than kTableLds, where too few waves fit a CU: then
-            // the bitmap of N bits per wave in HBM
-            constexpr size_t kTableLds = 40960;
+            // the bitmap of N bits per wave in HBM.  Long float rows in large
+            // batches are bound by their loads, which need more waves: there
+            // from 16 KiB on (4,000 queries of 10^5 x 960, degree 32, ef 64: 6.4 ms
+            // with up to 40 KiB, 5.0 so), and long lists beside the table
+            // leave fewer waves: from 20 KiB on (4,000 queries of 100,000 x
+            // 128 bytes, degree 32, ef 257: 5.4 and 4.0 ms; at degrees beyond
+            // 32 the bitmap's search for repeats within a row costs more:
+            // 3,000 x 20, degree 112, ef 700: 8.7 and 18.2 ms)
+            const bool loads_bound = a.lane_rows || (rows_dtype == GT_DTYPE_F32 && D > 448 && nq > 1024);
+            const size_t kTableLds = loads_bound ? 16384 : ef > 256 && degree <= 32 && nq > 1024 ? 20480 : 40960;
             int H = p.visited_slots;
             bool bitmap_only = H == -1;
             if (H == 0) {
-                const int64_t want = std::min<int64_t>(static_cast<int64_t>(degree) * ef * 10 / 9, N * 16 / 13 + 1);
+                // (long lists: room for 1.1 degree x ef, which no query was
+                // seen to outgrow: of 1,000 queries in 200,000 normal rows x
+                // 100, degree 16, ef 400, 11 did, 5.3 ms where the bitmap takes 3.0)
+                const int64_t visits = static_cast<int64_t>(degree) * ef;
+                const int64_t want = std::min<int64_t>(ef > 256 ? visits * 27 / 20 : visits * 10 / 9, N * 16 / 13 + 1);
                 const size_t spare = std::min<size_t>(kTableLds, 163840 / static_cast<size_t>(ceil_div(nq, 256)));
                 H = 512;
                 set_table(H);
                 while (H < want && search_query_lds(a, esz) <= kTableLds) set_table(H *= 2);
-                bitmap_only = search_query_lds(a, esz) > kTableLds;
+                // (short lists visit many points for their length: a query run
+                // again costs two whole chains)
+                bitmap_only = search_query_lds(a, esz) > kTableLds || (a.lane_rows && ef < 32);
                 while (!bitmap_only && H < 2 * want) {
                     set_table(2 * H);
                     if (search_query_lds(a, esz) > spare) break;

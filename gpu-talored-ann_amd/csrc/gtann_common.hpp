@@ -132,6 +132,7 @@ struct SearchArgs {
     int32_t buckets;          // visited table: 16-byte buckets (power of two); 0 = bitmap mode
     int32_t half;             // its entries: 1 = eight 16-bit per bucket, 0 = four ids
     int32_t nbits, lbits;     // bits of an id, of a bucket number
+    int32_t lane_rows;        // 1: float rows by a lane each
     int32_t vlimit;           // visited points beyond which the query is left to the bitmap
     uint32_t* bitmap;         // bitmap mode: gridDim.x slots of bm_words words, zero on entry
     int64_t bm_words;

@@ -92,6 +92,7 @@ __device__ __forceinline__ uint64_t wave_min_u64(uint64_t k)
 
 // Loads of a row that may start at any element
 typedef float f2u __attribute__((ext_vector_type(2), aligned(4)));
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
 typedef uint32_t u4u __attribute__((ext_vector_type(4), aligned(1)));
 typedef uint32_t u4a __attribute__((ext_vector_type(4)));
 
@@ -286,6 +287,7 @@ struct BestList {
 // (the query row padded to whole groups of eight quads)
 __host__ __device__ inline int search_query_bytes(int D, int esz) { return (D * esz + 127) / 128 * 128 + 16; }
 constexpr int kRowQuads = 32;      // quads of dimensions summed at a time (float rows)
+constexpr int kLaneQuads = 16;     // the same with a lane per row
 
 // x of the lane that CTRL names, within a row of 16 lanes
 template <int CTRL>
@@ -295,7 +297,12 @@ __device__ __forceinline__ int row_lane(int x)
 }
 
 // VS: the visited set (0 bitmap in HBM, 1 table of 16-bit entries, 2 table of ids)
-template <typename T, int R, int VS>
+// LANE: float rows by one lane each, up to 64 at a time, instead of two lanes
+// each, up to 32 (search_lane_rows).  A load of 16 bytes per lane instead of 8
+// asks the vector cache for half as many lines per row, which bounds many
+// queries over long rows; two lanes per row have half of the dependent sums
+// and registers for a whole row of 128 in flight, which bounds few.
+template <typename T, int R, int VS, bool LANE = false>
 __global__ void __attribute__((amdgpu_flat_work_group_size(64, 64), amdgpu_waves_per_eu(3))) graph_search_kernel(SearchArgs a)
 {
     constexpr bool INT = !std::is_same<T, float>::value;
@@ -546,6 +553,54 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(64, 64), amdgpu_waves
                         }
                     }
                 }
+            } else if constexpr (LANE) {
+                // rows past the last new point are not read (zeros)
+                const int n4 = D >> 2;
+                const bool on = lane < nn;
+                const float* row = X + static_cast<int64_t>(nid[min(lane, nn - 1)]) * a.ld;
+                const float* qr = reinterpret_cast<const float*>(qb);
+                float s[4] = {0.f, 0.f, 0.f, 0.f};
+                auto add = [&](float x, float y, float& acc) __attribute__((always_inline)) {
+                    const float t = y - x;
+                    acc = a.metric == 0 ? fmaf(t, t, acc) : fmaf(y, x, acc);
+                };
+                f4u x[kLaneQuads];
+#pragma unroll
+                for (int k = 0; k < kLaneQuads; ++k) x[k] = f4u{0.f, 0.f, 0.f, 0.f};
+                for (int q0 = 0; q0 < n4; q0 += kLaneQuads) {
+                    const f4u* xr = reinterpret_cast<const f4u*>(row) + q0;
+                    const int n = n4 - q0;
+                    if (on) {
+                        if (n >= kLaneQuads) {
+#pragma unroll
+                            for (int k = 0; k < kLaneQuads; ++k) x[k] = xr[k];
+                        } else {
+#pragma unroll
+                            for (int k = 0; k < kLaneQuads; ++k)
+                                if (k < n) x[k] = xr[k];
+                        }
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (last && q0 == 0) scan();
+                    const float4* yr = reinterpret_cast<const float4*>(qr) + q0;
+#pragma unroll
+                    for (int k = 0; k < kLaneQuads; ++k)
+                        if (k < n) {
+                            const float4 y = yr[k];
+                            add(x[k][0], y.x, s[0]);
+                            add(x[k][1], y.y, s[1]);
+                            add(x[k][2], y.z, s[2]);
+                            add(x[k][3], y.w, s[3]);
+                        }
+                }
+                for (int t = 0; t < (D & 3); ++t) {
+                    const float v = on ? row[4 * n4 + t] : 0.f;
+                    if (t == 0) add(v, qr[4 * n4], s[0]);
+                    else if (t == 1) add(v, qr[4 * n4 + 1], s[1]);
+                    else add(v, qr[4 * n4 + 2], s[2]);
+                }
+                const float d = (s[0] + s[1]) + (s[2] + s[3]);
+                if (on) ndv[lane] = a.metric == 0 ? d : -d;
             } else {
                 const int n4 = D >> 2;
                 for (int base = 0; base < nn; base += 32) {
@@ -773,6 +828,17 @@ void launch_search_totals_init(SearchTotals* t, hipStream_t s)
     GT_HIP(hipGetLastError());
 }
 
+// Whether a launch reads float rows a lane each.  10,000 queries of 10^5 x 960
+// (ef 64 / 200), times of two lanes per row and one, degree 16: 10.5 / 28.7 and
+// 8.6 / 29.6 ms; 32: 14.7 / 38.8 and 10.2 / 34.1; 48: 21.5 / 52.3 and 13.0 /
+// 37.4; x 300, degree 32: 3.5 / 10.3 and 3.7 / 13.6, 48: 5.3 / 17.7 and 5.0 /
+// 15.3.  1,000 queries (fewer than SIMDs), x 960, degree 32: 1.66 / 4.2 and
+// 2.3 / 6.0, 48: 2.5 / 6.1 and 2.4 / 6.7.
+bool search_lane_rows(int64_t queries, int D, int degree, bool floats)
+{
+    return floats && queries > 1024 && ((D > 448 && degree > 16) || (D > 256 && degree > 32));
+}
+
 // LDS bytes of one query of the launch a.
 size_t search_query_lds(const SearchArgs& a, int esz)
 {
@@ -791,6 +857,22 @@ static void launch_search_t(const SearchArgs& a, unsigned grid, hipStream_t s)
                                        static_cast<int>(lds)));
         hipLaunchKernelGGL(kernel, dim3(grid), dim3(64), lds, s, a);
     };
+    if constexpr (std::is_same<T, float>::value) {
+        if (a.lane_rows) {
+            if (a.buckets == 0) {
+                if (a.ef <= 256) go(&graph_search_kernel<T, 4, 0, true>);
+                else go(&graph_search_kernel<T, 0, 0, true>);
+            } else if (a.half) {
+                if (a.ef <= 256) go(&graph_search_kernel<T, 4, 1, true>);
+                else go(&graph_search_kernel<T, 0, 1, true>);
+            } else {
+                if (a.ef <= 256) go(&graph_search_kernel<T, 4, 2, true>);
+                else go(&graph_search_kernel<T, 0, 2, true>);
+            }
+            GT_HIP(hipGetLastError());
+            return;
+        }
+    }
     // the best list in registers where four per lane hold it
     if (a.buckets == 0) {
         if (a.ef <= 256) go(&graph_search_kernel<T, 4, 0>);

@@ -334,7 +334,8 @@ typedef struct gt_search_params {
     uint64_t seed;          /* entry draw when `entries` is NULL */
     int32_t visited_slots;  /* visited set per query: 0 = automatic (an on-chip hash table, or an HBM
                                bitmap of N bits per wave when the query would take more than 40 KiB
-                               of LDS with it); -1 = the HBM bitmap; else the on-chip table's slots (power of
+                               of LDS with it, or 16 to 20 KiB for long float rows or lists of
+                               more than 256 points in calls of more than 1,024 queries); -1 = the HBM bitmap; else the on-chip table's slots (power of
                                two >= 512), a query that outgrows it run again with the bitmap */
     int32_t reserved_;
 } gt_search_params;

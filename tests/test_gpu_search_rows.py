@@ -88,3 +88,26 @@ def test_base_at_an_odd_address(ctx, dtype):
     rid, rd, _ = O.search(X.astype(np.float32), g, Q.astype(np.float32), ent, 5, 32)
     np.testing.assert_array_equal(ids.cpu().numpy(), rid)
     np.testing.assert_array_equal(d.cpu().numpy().view(np.uint32), rd.view(np.uint32))
+
+
+@pytest.mark.parametrize("metric", ["l2", "ip"])
+@pytest.mark.parametrize("D,deg,ef", [(257, 33, 64), (449, 17, 1), (322, 64, 63), (323, 65, 65), (384, 130, 20), (703, 20, 256),
+                                      (960, 48, 257), (1024, 32, 40), (321, 33, 128)])
+def test_many_queries_over_long_rows(ctx, D, deg, ef, metric):
+    """Calls of more than 1,024 queries read float rows beyond 256 dimensions a
+    lane each: the restatement's results, and those of the same queries in
+    smaller calls."""
+    rng = np.random.default_rng(D + deg)
+    X, g, Q, ent = _case(rng, 700, D, np.float32, deg, 1029)
+    print(f"search long rows D={D} deg={deg} ef={ef} {metric}", flush=True)
+    k = min(ef, 5)
+    _compare(ctx, X, g, Q, ent, k, ef, metric=metric)
+    big = ctx.search(X, g, Q, topk=k, ef=ef, entries=ent, metric=metric)
+    for s in (slice(0, 600), slice(600, 1029)):
+        part = ctx.search(X, g, Q[s], topk=k, ef=ef, entries=ent[s], metric=metric)
+        np.testing.assert_array_equal(part[0], big[0][s])
+        np.testing.assert_array_equal(part[1].view(np.uint32), big[1][s].view(np.uint32))
+    for slots in (-1, 512):
+        out = ctx.search(X, g, Q, topk=k, ef=ef, entries=ent, metric=metric, visited_slots=slots)
+        np.testing.assert_array_equal(out[0], big[0])
+        np.testing.assert_array_equal(out[1].view(np.uint32), big[1].view(np.uint32))

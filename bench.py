@@ -11,7 +11,8 @@ with the dataset already resident in HBM.  Prints one JSON line.
 knn_select_kernel when the rows are integers, as C2's are;
 knn_f32_collect_kernel + knn_select_kernel for float rows up to 160
 dimensions, behind the fp16 screen (knn_screen_kernel) on passes of at least
-2^27 pairs; knn_wide_kernel beyond): achieved = the algorithmic ops of its launches
+2^27 pairs; knn_wide_collect_kernel + knn_sort_select_kernel beyond 256
+dimensions, on the bf16 matrix cores): achieved = the algorithmic ops of its launches
 (2*D per scanned (query, pool row) pair) over their summed duration, both
 measured by the library with HIP events on its stream.  `traffic` is read
 from profiles/<kernel>_<config>_traffic.json (knn_i8_collect_C2_traffic.json
@@ -56,6 +57,7 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, os.path.join(ROOT, "gpu-talored-ann_amd"))
 
 PEAK_FP32_MFMA = 157.3e12   # MI355X dense fp32 matrix, FLOP/s
+PEAK_BF16_MFMA = 2.5e15     # MI355X dense bf16 matrix, FLOP/s
 PEAK_INT8_MFMA = 5.0e15     # MI355X dense int8 matrix, OP/s
 PEAK_HBM = 8.0e12           # MI355X HBM3E, B/s
 
@@ -209,7 +211,10 @@ def knn_roofline(s, D, metric, M=64):
     the fp16 screen (knn_screen_kernel) first computes every pair of each
     work item on the fp16 matrix cores and the fp32 collect kernel then
     scans only the item's union of rows that can reach a list: there
-    `pairs_executed_share` is the share of pairs left to the fp32 MFMAs."""
+    `pairs_executed_share` is the share of pairs left to the fp32 MFMAs.
+    Rows beyond 256 dimensions in buckets of 400 or more are split into three
+    bf16 parts: six bf16 products per element, which `ops_executed_per_launch`
+    and `frac_executed` count."""
     launches = max(1, int(round(s["knn_launches"])))
     launch_s = s["t_knn"] / launches
     flops = s["knn_flops"] / launches
@@ -230,6 +235,10 @@ def knn_roofline(s, D, metric, M=64):
         peak, unit = PEAK_FP32_MFMA, "TFLOP/s"
         if done < pairs and 4 < M <= 64 and dp <= 160:   # the fp16 screen ran
             kname = f"knn_screen_kernel<{dp}, {mip}> (fp16) + " + kname
+    elif 4 < M <= 128 and float(s.get("max_bucket", 0.0)) >= 400:
+        kname = f"knn_wide_collect_kernel<{mip}> + " + ("knn_sort_select_kernel" if M > 64 else "knn_select_kernel")
+        peak, unit = PEAK_BF16_MFMA, "TFLOP/s"
+        executed *= 6
     else:
         kname, peak, unit = f"knn_wide_kernel<{mip}>", PEAK_FP32_MFMA, "TFLOP/s"
     return {"kernel": kname, "bound": "mfma", "achieved": flops / launch_s / 1e12, "peak": peak / 1e12,

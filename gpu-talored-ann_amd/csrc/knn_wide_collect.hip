@@ -38,14 +38,16 @@
 // per wave).  Short launches take 4 waves and 128 queries
 // (wide_queries_per_block).  A copy of the three parts, 6 bytes per element, was
 // slower: bucketed pass below 13.0 ms, build 187.
-// What bounds it (bucketed pass over 100,003 x 960, 25 buckets, one probe, M
-// 96; counters): where a CU has a block, its matrix cores are busy 57 % of the
-// time; they wait for the sums' 32 additions per tile, the split and the
-// barrier of each chunk.  Over the launch 30 %: some 400 blocks, a bucket's on
-// one XCD, hold the 256 CUs 52 % of the time.
-// Measured: that pass 20.3 ms on the fp32 kernel, 12.4 here; a 10^6 x 960
-// build 241 -> 172 ms; exact 100-NN of 10,000 queries in 1,000,003 x 100:
-// 40.3 -> 20.1 ms.  (With two fp16 parts, which lose bits: 8.4, 128 and 13.8.)
+// What bounds it (a 10^6 x 960 build, counters): six products per element at
+// 963 TFLOP/s, 85 % of what a large bf16 product reaches on the card (1.13
+// PFLOP/s); the matrix cores are busy 54 % of the time, beside the sums' 32
+// additions per tile, the split and the barrier of each chunk.  A pass of some
+// 400 blocks, a bucket's on one XCD, holds the CUs only 52 % of the time.
+// Measured: bucketed pass over 100,003 x 960 (25 buckets, one probe, M 96)
+// 20.8 ms on the fp32 kernel, 12.4 to 15.0 here (by GPU); the build 237 -> 166
+// to 172 ms; exact 100-NN of 10,000 queries in 1,000,003 x 100 40.2 -> 19.3 ms.
+// (With two fp16 parts, which lose bits: 8.4, 128 and 13.8.)
+//
 // Keys at or below a query's threshold go to its candidate slots in HBM as in
 // knn_collect.hip.  An unseeded pass first bounds each query's M-th smallest
 // key by bisection over the 192 keys of the first pool tile, which the lane

@@ -47,9 +47,10 @@ def test_slices_match_the_fp32_kernels(ctx, n, d, nq, k, distinct):
 @pytest.mark.parametrize("metric", ["l2", "ip"])
 @pytest.mark.parametrize("d", [33, 128, 300])
 def test_lists_do_not_depend_on_the_batch(ctx, d, metric):
+    # (5,003 queries: blocks of 256 queries and 8 waves; the smaller calls: 128 and 4)
     rng = np.random.default_rng(d)
-    X = rng.standard_normal((20011, d)).astype(np.float32)
-    q = rng.permutation(20011)[:3000]
+    X = rng.standard_normal((30011, d)).astype(np.float32)
+    q = rng.permutation(30011)[:5003]
     ids, dist = ctx.knn_exact(X, 20, queries=q, metric=metric)
     for nq in (1, 2, 33, 128, 255, 256, 700):
         i, v = ctx.knn_exact(X, 20, queries=q[:nq], metric=metric)

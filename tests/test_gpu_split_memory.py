@@ -1,7 +1,7 @@
 """Device memory and the rows kept for the split (bucketed kNN beyond 256
 dimensions): what a call returns does not depend on how much is free, a call
 whose copy does not fit still runs, and the copy is given back where another
-call needs its room.  The memory is taken by a tensor, never to the last: every
+call needs its room.  The memory is taken by tensors, never to the last: every
 case leaves half a GiB or more."""
 import numpy as np
 import pytest
@@ -34,12 +34,13 @@ def fresh():
 
 
 def _take(leave):
-    """A tensor over all of the free memory but `leave` bytes."""
+    """Tensors over all of the free memory but `leave` bytes."""
     import torch
     torch.cuda.empty_cache()
     free, _ = torch.cuda.mem_get_info()
     print(f"free {free >> 20} MiB, leaving {leave >> 20}", flush=True)
-    return torch.empty(free - leave, dtype=torch.uint8, device="cuda")
+    sizes = [32 << 30] * ((free - leave) >> 35) + [(free - leave) & ((32 << 30) - 1)]
+    return [torch.empty(n, dtype=torch.uint8, device="cuda") for n in sizes if n > 0]
 
 
 def _run(c, rows):
